@@ -288,9 +288,8 @@ __device__ __forceinline__ float rk4_step_c(const TraceArgs &a, const Cell &C, f
 // on five z-planes only (tz = 0, 1/4, 1/2, 3/4, 1), so the cell polynomial is
 // reduced to each plane's bilinear form once (ZP: 4 FMAs per coefficient
 // pair, none at tz = 0) and every stage evaluates that bilinear form (3 FMAs
-// per channel).  Whether every stage point lies in the cell is tracked as the
-// running min / max of tx, ty over the stages (two v_min3 / v_max3 per stage)
-// and tested once per step.
+// per channel).  Whether every stage point lies in the cell is tracked as a
+// running maximum over the stages and tested once per step.
 // ---------------------------------------------------------------------------
 struct ZP {
     float4 A, B, Cc, E;  // f = A + B tx + Cc ty + E tx ty on one z-plane
@@ -307,10 +306,9 @@ struct ZP {
 // more than that between stages is redone exactly.
 template <bool VF, bool SEED = false>
 __device__ __forceinline__ void rhs_z(const TraceArgs &a, const ZP &z, float ox, float oy, const State &s, float4 &g,
-                                      float &iW, float &vf, float &mn, float &mx, float &e) {
+                                      float &iW, float &vf, uint32_t &far, float &e) {
     const float tx = fmaf(a.sx, s.qx, ox), ty = fmaf(a.sy, s.qy, oy);
-    mn = fminf(mn, fminf(tx, ty));
-    mx = fmaxf(mx, fmaxf(tx, ty));
+    far = max(far, max(__float_as_uint(tx), __float_as_uint(ty)));
     g = f4fma(f4fma(z.E, ty, z.B), tx, f4fma(z.Cc, ty, z.A));
     const float W = 1.0f + s.Wd;
     if (SEED) {
@@ -324,7 +322,8 @@ __device__ __forceinline__ void rhs_z(const TraceArgs &a, const ZP &z, float ox,
 
 // the largest stage-to-stage relative change of W a cached step may have
 // (the Newton-refined 1 / W is then exact to fp32 rounding)
-constexpr float kNewtonTolInv = 4096.0f;
+constexpr float kNewtonTol = 1.0f / 4096.0f;
+constexpr uint32_t kInCell = 0x3f800000u;  // the bit pattern of 1
 
 // y + c r, r the unscaled right-hand side of stage state s with field g
 template <bool TAU>
@@ -338,34 +337,53 @@ __device__ __forceinline__ State axpy_r(const State &y, float c, const State &s,
 // phase is summed by the composite Simpson rule over the march's lattice
 // points (march_m2), so only the first stage needs the Phi channel and the
 // others' Phi (and the Phi channel of the zm and z1 planes) is never formed.
-// mn / mx collect the stage points' in-cell coordinates, and mx also
-// 4096 x the largest relative change of W between stages: the step is good
-// from the cache only if mn >= 0 and mx <= 1.  iWc: in, 1 / W of a state near
-// the start (the previous step's last stage, or exact); out, the last
-// stage's 1 / W, the next step's seed.
+// The step is good from the cache only if every stage point lies in the cell
+// (far <= kInCell) and W changed by at most kNewtonTol between stages (em, the
+// largest relative change); else it is redone by gathers.  far is one unsigned
+// maximum of the bit patterns of the stage points' in-cell coordinates: one in
+// [0, 1] is at most the pattern of 1, and a negative one (sign bit) or a NaN is
+// above it, so one v_max3_u32 per stage tests both bounds of both coordinates
+// where a running minimum and maximum took two.
+// iWc: in, 1 / W of a state near the start (the previous step's last stage,
+// or exact); out, the last stage's 1 / W, the next step's seed.
 template <bool TAU>
 __device__ __forceinline__ float rk4_half_z(const TraceArgs &a, const ZP &z0, const ZP &zm, const ZP &z1, float ox,
-                                            float oy, State &y, float &mn, float &mx, float &iWc) {
+                                            float oy, State &y, float &iWc, uint32_t &far, float &em) {
     // the new state is accumulated as y + h/6 (k1 + 2 k2 + 2 k3 + k4) stage
     // by stage, each weight folded into that stage's factor c / W
     constexpr float h6 = 0.5f / 6.0f, h3 = 0.5f / 3.0f;
     float4 g;
     float iW = iWc, vf = 0.f, unused, e1, e2, e3, e4;
-    rhs_z<true, true>(a, z0, ox, oy, y, g, iW, vf, mn, mx, e1);
+    far = 0u;
+    rhs_z<true, true>(a, z0, ox, oy, y, g, iW, vf, far, e1);
     const float phi = g.w * vf;
     State yn = axpy_r<TAU>(y, h6 * iW, y, g);
     const State s2 = axpy_r<TAU>(y, 0.25f * iW, y, g);
-    rhs_z<false, true>(a, zm, ox, oy, s2, g, iW, unused, mn, mx, e2);
+    rhs_z<false, true>(a, zm, ox, oy, s2, g, iW, unused, far, e2);
     yn = axpy_r<TAU>(yn, h3 * iW, s2, g);
     const State s3 = axpy_r<TAU>(y, 0.25f * iW, s2, g);
-    rhs_z<false, true>(a, zm, ox, oy, s3, g, iW, unused, mn, mx, e3);
+    rhs_z<false, true>(a, zm, ox, oy, s3, g, iW, unused, far, e3);
     yn = axpy_r<TAU>(yn, h3 * iW, s3, g);
     const State s4 = axpy_r<TAU>(y, 0.5f * iW, s3, g);
-    rhs_z<false, true>(a, z1, ox, oy, s4, g, iW, unused, mn, mx, e4);
+    rhs_z<false, true>(a, z1, ox, oy, s4, g, iW, unused, far, e4);
     y = axpy_r<TAU>(yn, h6 * iW, s4, g);
     iWc = iW;
-    mx = fmaxf(mx, kNewtonTolInv * fmaxf(fmaxf(fabsf(e1), fabsf(e2)), fmaxf(fabsf(e3), fabsf(e4))));
+    em = fmaxf(fmaxf(fabsf(e1), fabsf(e2)), fmaxf(fabsf(e3), fabsf(e4)));
     return phi;
+}
+
+// the plane forms z0, D below from a cell's eight nodes
+__device__ __forceinline__ void planes_of(const float4 &c000, const float4 &c100, const float4 &c010, const float4 &c110,
+                                          const float4 &c001, const float4 &c101, const float4 &c011,
+                                          const float4 &c111, ZP &z0, ZP &D) {
+    z0.A = c000;
+    z0.B = f4sub(c100, c000);
+    z0.Cc = f4sub(c010, c000);
+    z0.E = f4sub(f4sub(c110, c010), z0.B);
+    D.A = f4sub(c001, c000);
+    D.B = f4sub(f4sub(c101, c001), z0.B);
+    D.Cc = f4sub(f4sub(c011, c001), z0.Cc);
+    D.E = f4sub(f4sub(f4sub(c111, c011), f4sub(c101, c001)), z0.E);
 }
 
 // The cell as plane forms: z0 on its lower z-plane and D = (upper - lower),
@@ -385,16 +403,7 @@ __device__ __forceinline__ void load_planes(const TraceArgs &A, int ix, int iy, 
     }
     const int64_t plane = (int64_t)A.nx * A.ny;
     const float4 *p = A.field + node_index(A, ix, iy, iz);
-    const float4 c000 = p[0], c100 = p[1], c010 = p[A.nx], c110 = p[A.nx + 1];
-    const float4 c001 = p[plane], c101 = p[plane + 1], c011 = p[plane + A.nx], c111 = p[plane + A.nx + 1];
-    z0.A = c000;
-    z0.B = f4sub(c100, c000);
-    z0.Cc = f4sub(c010, c000);
-    z0.E = f4sub(f4sub(c110, c010), z0.B);
-    D.A = f4sub(c001, c000);
-    D.B = f4sub(f4sub(c101, c001), z0.B);
-    D.Cc = f4sub(f4sub(c011, c001), z0.Cc);
-    D.E = f4sub(f4sub(f4sub(c111, c011), f4sub(c101, c001)), z0.E);
+    planes_of(p[0], p[1], p[A.nx], p[A.nx + 1], p[plane], p[plane + 1], p[plane + A.nx], p[plane + A.nx + 1], z0, D);
 }
 
 // the plane dt above plane z (D = the cell's upper-minus-lower plane form)
@@ -429,17 +438,26 @@ __device__ __forceinline__ void ledger_first(PhaseLedger &L, double &ph, float p
     ph += (double)add;
 }
 
+// the cell's second step when both of its steps ran from the cache
+__device__ __forceinline__ void ledger_smooth(PhaseLedger &L, double &ph, float phi) {
+    constexpr float k6 = 1.0f / 6.0f;
+    const float add = k6 * fmaf(4.0f, phi, L.phi0);
+    L.pend = k6;
+    ph += (double)add;
+}
+
 // the cell's second step (odd k) from state ys0 (its start) to ys1 (its end)
 __device__ __forceinline__ void ledger_second(const TraceArgs &a, float pxb, float pyb, int k, PhaseLedger &L,
                                               double &ph, float phi, bool smooth, float dph, const State &ys0,
                                               const State &ys1) {
-    constexpr float k6 = 1.0f / 6.0f, k12 = 1.0f / 12.0f;
+    constexpr float k12 = 1.0f / 12.0f;
     const float Zh = (float)k * 0.5f;  // the cell's half plane
     float add;
     if (L.s1 && smooth) {
-        add = k6 * fmaf(4.0f, phi, L.phi0);
-        L.pend = k6;
-    } else if (L.s1) {  // the first half took the cache, this one crossed a face
+        ledger_smooth(L, ph, phi);
+        return;
+    }
+    if (L.s1) {  // the first half took the cache, this one crossed a face
         const float pm = phi_at(a, pxb, pyb, Zh - 0.25f, ys0, 0.25f);
         add = k12 * (L.phi0 + fmaf(4.0f, pm, phi)) + dph;
         L.pend = 0.f;
@@ -501,7 +519,8 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
     };
     while (k < K) {
         State yn;
-        float phi;
+        float phi, em;
+        uint32_t far;
         bool ok;
         if (k & 1) {  // the second step of a cell whose first step was redone
             int ix, iy;
@@ -513,13 +532,12 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
             }
             ZP z0, D;
             load_planes<FORMS>(a, ix, iy, k >> 1, z0, D);
-            float mn = inside ? 0.f : -1.f, mx = 0.f;
             const ZP zh = zstep(z0, 0.5f, D);
             const ZP z3 = zstep(zh, 0.25f, D);
             const ZP z1 = zstep(z3, 0.25f, D);
             yn = ys;
-            phi = rk4_half_z<TAU>(a, zh, z3, z1, ox, oy, yn, mn, mx, iWc);
-            ok = mn >= 0.f && mx <= 1.f;
+            phi = rk4_half_z<TAU>(a, zh, z3, z1, ox, oy, yn, iWc, far, em);
+            ok = far <= kInCell && em <= kNewtonTol && inside;
         } else {  // whole cells from the cache
             bool done = false;
             for (;;) {
@@ -532,12 +550,11 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
                 ZP z0, D;
                 load_planes<FORMS>(a, ix, iy, k >> 1, z0, D);
                 __builtin_amdgcn_s_setprio(0);
-                float mn = inside ? 0.f : -1.f, mx = 0.f;
                 const ZP zq = zstep(z0, 0.25f, D);
                 const ZP zh = zstep(z0, 0.5f, D);
                 yn = ys;
-                phi = rk4_half_z<TAU>(a, z0, zq, zh, ox, oy, yn, mn, mx, iWc);
-                ok = mn >= 0.f && mx <= 1.f;
+                phi = rk4_half_z<TAU>(a, z0, zq, zh, ox, oy, yn, iWc, far, em);
+                ok = far <= kInCell && em <= kNewtonTol && inside;
                 if (__ballot(!ok) != 0) break;  // redo the cell's first step below
                 ys = yn;
                 ledger_first(L, ph, phi, true, 0.f);
@@ -546,8 +563,8 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
                 const ZP z3 = zstep(zh, 0.25f, D);
                 const ZP z1 = zstep(z3, 0.25f, D);
                 yn = ys;
-                phi = rk4_half_z<TAU>(a, zh, z3, z1, ox, oy, yn, mn, mx, iWc);
-                ok = mn >= 0.f && mx <= 1.f;
+                phi = rk4_half_z<TAU>(a, zh, z3, z1, ox, oy, yn, iWc, far, em);
+                ok = far <= kInCell && em <= kNewtonTol && inside;
                 if (__ballot(!ok) != 0) break;  // redo the cell's second step below
                 ledger_second(a, pxb, pyb, k, L, ph, phi, true, 0.f, ys, yn);
                 ys = yn;
@@ -578,6 +595,171 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
     }
     if (L.pend != 0.f) ph += (double)(L.pend * phi_at(a, pxb, pyb, (float)K * 0.5f, ys));  // exit point
     return good && !crossed && lateral_inside(a, pxb, pyb, ys) == in0;
+}
+
+// The h = 1/2 march of a wave whose rays are all at the same step (a beam
+// launched from one plane: every ray of it), what march_m2 does for lanes at
+// different steps, bit for bit.  With one step counter for the wave the loops
+// are scalar, the lanes' conditions are 64-bit masks in scalar registers and
+// the cell's address is a scalar row base plus one 32-bit lane offset; each
+// step ends in the state registers the next one starts from.  The march is
+// bound by VALU issue, and all of that is VALU work march_m2 does per cell:
+// 64-bit lane addresses, selects for the lanes outside the grid, compares
+// turned into integers for the ballots, copies on the loop's back edge (405 ->
+// 360 VALU per cell; 1e7 rays: 35.3 -> 32.7 ms through 512^3, 95.9 -> 91.4 ms
+// through 1024^3, where more steps are redone by gathers; 1e5 rays through
+// 128^3: 206 -> 187 us).  The offset (16 or 64 bytes a node) and the row index are exact in 32 bits and in
+// fp32 while nx ny <= 2^24, hence kUniformPlane.
+constexpr uint32_t kUniformPlane = 1u << 24;
+
+// lane mask -> this lane's condition
+__device__ __forceinline__ bool lane_of(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+__device__ __forceinline__ uint64_t mask_of(bool c) { return __builtin_amdgcn_ballot_w64(c); }
+
+// The cell of the current position: its byte offset in a plane (off, from the
+// row index computed exactly in fp32), the entry point relative to it, and the
+// lanes whose position lies in the grid.  A position outside is clamped to the
+// nearest cell (its step is redone by gathers); kClampBelow keeps the last
+// node in the last cell.
+template <bool FORMS>
+__device__ __forceinline__ uint64_t locate_u(const TraceArgs &a, float pxb, float pyb, float cx, float cy, float fnx,
+                                             const State &s, float &ox, float &oy, uint32_t &off) {
+    const float px = fmaf(a.sx, s.qx, pxb), py = fmaf(a.sy, s.qy, pyb);
+    const float ix = floorf(__builtin_amdgcn_fmed3f(px, 0.f, cx)), iy = floorf(__builtin_amdgcn_fmed3f(py, 0.f, cy));
+    ox = pxb - ix;
+    oy = pyb - iy;
+    off = (uint32_t)fmaf(iy, fnx, ix) * (FORMS ? 64u : 16u);
+    return mask_of(__float_as_uint(px) <= __float_as_uint(a.fx1)) & mask_of(__float_as_uint(py) <= __float_as_uint(a.fy1));
+}
+
+// load_planes from the address of node (0, 0) of the cell's lower plane, the
+// bytes from row to row and plane to plane, and the lane's offset.  The
+// pointers are to global memory by type: a batch item's come from memory,
+// where the compiler could not tell and would emit flat loads.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) char *gbytes;
+__device__ __forceinline__ float4 gload4(gbytes p) {
+    const f32x4 v = *reinterpret_cast<const __attribute__((address_space(1))) f32x4 *>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+template <bool FORMS>
+__device__ __forceinline__ void load_planes_u(gbytes base, int64_t row, int64_t step, uint32_t off, ZP &z0, ZP &D) {
+    const gbytes p0 = base + off, q0 = base + step + off;
+    if (FORMS) {
+        z0 = ZP{gload4(p0), gload4(p0 + 16), gload4(p0 + 32), gload4(p0 + 48)};
+        D = ZP{f4sub(gload4(q0), z0.A), f4sub(gload4(q0 + 16), z0.B), f4sub(gload4(q0 + 32), z0.Cc),
+               f4sub(gload4(q0 + 48), z0.E)};
+        return;
+    }
+    const gbytes p1 = base + row + off, q1 = base + step + row + off;
+    planes_of(gload4(p0), gload4(p0 + 16), gload4(p1), gload4(p1 + 16), gload4(q0), gload4(q0 + 16), gload4(q1),
+              gload4(q1 + 16), z0, D);
+}
+
+template <bool TAU, bool FORMS>
+__device__ __forceinline__ bool march_m2u(const TraceArgs &a, float pxb, float pyb, int k, int K, State &ys,
+                                          double &ph) {
+    const uint64_t act = mask_of(true);
+    const uint64_t in0 = mask_of(lateral_inside(a, pxb, pyb, ys));
+    uint64_t good = act, crossed = 0ull;
+    if (k < K && (k & 1)) {
+        ph += (double)rk4_step(a, pxb, pyb, (float)k * 0.5f, 0.5f, ys);
+        good = mask_of(ys.Wd > kWdMin);
+        ++k;
+    }
+    if (k < K) {
+        constexpr int NB = FORMS ? 64 : 16;
+        const float cx = __uint_as_float(__float_as_uint(a.fx1) - 1u), cy = __uint_as_float(__float_as_uint(a.fy1) - 1u);
+        const float fnx = (float)a.nx;
+        // bytes from plane to plane and row to row
+        const int64_t step = (int64_t)a.plane * NB, row = (int64_t)a.nx * NB;
+        gbytes base = (gbytes)(FORMS ? a.forms : a.field) + (k >> 1) * step;
+        PhaseLedger L;
+        float iWc = __builtin_amdgcn_rcpf(1.0f + ys.Wd);
+        for (;;) {
+            float ox, oy, phi, em;
+            uint32_t off, far;
+            uint64_t in, okm;
+            State yn;
+            // whole cells from the cache
+            for (;;) {
+                ZP z0, D;
+                // raised wave priority while the cell's loads are issued (march_m2)
+                __builtin_amdgcn_s_setprio(1);
+                in = locate_u<FORMS>(a, pxb, pyb, cx, cy, fnx, ys, ox, oy, off);
+                load_planes_u<FORMS>(base, row, step, off, z0, D);
+                __builtin_amdgcn_s_setprio(0);
+                crossed |= in ^ in0;
+                const ZP zq = zstep(z0, 0.25f, D);
+                const ZP zh = zstep(z0, 0.5f, D);
+                yn = ys;
+                phi = rk4_half_z<TAU>(a, z0, zq, zh, ox, oy, yn, iWc, far, em);
+                okm = mask_of(far <= kInCell) & mask_of(em <= kNewtonTol) & in;
+                if (__builtin_expect(okm != act, 0)) break;
+                ledger_first(L, ph, phi, true, 0.f);
+                good &= mask_of(yn.Wd > kWdMin);
+                ys = yn;
+                ++k;
+                const ZP z3 = zstep(zh, 0.25f, D);
+                const ZP z1 = zstep(z3, 0.25f, D);
+                phi = rk4_half_z<TAU>(a, zh, z3, z1, ox, oy, yn, iWc, far, em);
+                okm = mask_of(far <= kInCell) & mask_of(em <= kNewtonTol) & in;
+                if (__builtin_expect(okm != act, 0)) break;
+                ledger_smooth(L, ph, phi);
+                good &= mask_of(yn.Wd > kWdMin);
+                ys = yn;
+                ++k;
+                base += step;
+                if (k >= K) break;
+            }
+            // the three ways out of that loop meet here: hidden from the compiler,
+            // which would otherwise give each its own copy of what follows and
+            // pay for it with register copies on the loop's common path
+            asm volatile("" : "+s"(okm), "+s"(k));
+            if (okm == act) break;  // k >= K
+            // a lane left its cell in step k: those lanes redo it with gathers
+            for (;;) {
+                float dph = 0.f;
+                const bool ok = lane_of(okm);
+                if (!ok) {
+                    yn = ys;
+                    phi = rk4_step_phi(a, pxb, pyb, (float)k * 0.5f, 0.5f, yn, dph);
+                    iWc = __builtin_amdgcn_rcpf(1.0f + yn.Wd);  // an exact seed after a gathered step
+                }
+                if (k & 1)
+                    ledger_second(a, pxb, pyb, k, L, ph, phi, ok, dph, ys, yn);
+                else
+                    ledger_first(L, ph, phi, ok, dph);
+                ys = yn;
+                good &= mask_of(ys.Wd > kWdMin);
+                ++k;
+                if (!(k & 1)) break;
+                // the cell's second step: the lanes that redid the first one
+                // locate the cell they are in now, the others reload their own
+                float ox2, oy2;
+                uint32_t off2;
+                const uint64_t in2 = locate_u<FORMS>(a, pxb, pyb, cx, cy, fnx, ys, ox2, oy2, off2);
+                crossed |= (in2 ^ in0) & ~okm;
+                in = (in & okm) | (in2 & ~okm);
+                ox = ok ? ox : ox2;
+                oy = ok ? oy : oy2;
+                off = ok ? off : off2;
+                ZP u0, uD;
+                load_planes_u<FORMS>(base, row, step, off, u0, uD);
+                const ZP uh = zstep(u0, 0.5f, uD);
+                const ZP u3 = zstep(uh, 0.25f, uD);
+                const ZP u1 = zstep(u3, 0.25f, uD);
+                phi = rk4_half_z<TAU>(a, uh, u3, u1, ox, oy, yn, iWc, far, em);
+                okm = mask_of(far <= kInCell) & mask_of(em <= kNewtonTol) & in;
+            }
+            base += step;
+            if (k >= K) break;
+        }
+        if (L.pend != 0.f) ph += (double)(L.pend * phi_at(a, pxb, pyb, (float)K * 0.5f, ys));  // exit point
+    }
+    const bool in1 = lateral_inside(a, pxb, pyb, ys);
+    return lane_of(good & ~crossed & ~(mask_of(in1) ^ in0)) && ys.Wd > kWdMin;
 }
 
 // Steps k .. K-1 (z = k h) from the lattice, cell-cached.  Every lane loads
@@ -673,16 +855,24 @@ __device__ __forceinline__ void trace_ray(const TraceArgs &a, int64_t t) {
             py += (double)a.sy * V0 / W0 * d;
             tau += a.dz * d / W0;
         } else {
-            const float pxb = (float)px, pyb = (float)py;
+            // + 0: never -0, whose bit pattern the cell tests would take for a negative coordinate
+            const float pxb = (float)px + 0.f, pyb = (float)py + 0.f;
             const int K = (a.nz - 1) * a.m;
             const int kstart = (int)ceil(Zs * a.m - 1e-9);
             const double h0 = kstart * (double)a.h - Zs;
             if (CACHED) {
                 // partial first step (off-lattice start) with gathers, then the lattice
                 if (h0 > 1e-12) ph += (double)rk4_step(a, pxb, pyb, (float)Zs, (float)h0, ys);
-                if (!(M2 ? march_m2<TAU, FORMS>(a, pxb, pyb, kstart, K, ys, ph)
-                         : march_cached<TAU>(a, pxb, pyb, kstart, K, ys, ph)))
-                    st = 1;
+                bool stays;
+                if (M2) {
+                    const int ku = __builtin_amdgcn_readfirstlane(kstart);
+                    stays = a.plane <= kUniformPlane && mask_of(kstart != ku) == 0
+                                ? march_m2u<TAU, FORMS>(a, pxb, pyb, ku, K, ys, ph)
+                                : march_m2<TAU, FORMS>(a, pxb, pyb, kstart, K, ys, ph);
+                } else {
+                    stays = march_cached<TAU>(a, pxb, pyb, kstart, K, ys, ph);
+                }
+                if (!stays) st = 1;
             } else {
                 if (h0 > 1e-12) ph += (double)rk4_step(a, pxb, pyb, (float)Zs, (float)h0, ys);
                 const bool in0 = lateral_inside(a, pxb, pyb, ys);
