@@ -305,9 +305,9 @@ struct ZP {
 // rounding while |e| <= 2^-12; e is returned so that a step whose W changed
 // more than that between stages is redone exactly.
 template <bool VF, bool SEED = false>
-__device__ __forceinline__ void rhs_z(const TraceArgs &a, const ZP &z, float ox, float oy, const State &s, float4 &g,
+__device__ __forceinline__ void rhs_z(float sx, float sy, const ZP &z, float ox, float oy, const State &s, float4 &g,
                                       float &iW, float &vf, uint32_t &far, float &e) {
-    const float tx = fmaf(a.sx, s.qx, ox), ty = fmaf(a.sy, s.qy, oy);
+    const float tx = fmaf(sx, s.qx, ox), ty = fmaf(sy, s.qy, oy);
     far = max(far, max(__float_as_uint(tx), __float_as_uint(ty)));
     g = f4fma(f4fma(z.E, ty, z.B), tx, f4fma(z.Cc, ty, z.A));
     const float W = 1.0f + s.Wd;
@@ -347,7 +347,7 @@ __device__ __forceinline__ State axpy_r(const State &y, float c, const State &s,
 // iWc: in, 1 / W of a state near the start (the previous step's last stage,
 // or exact); out, the last stage's 1 / W, the next step's seed.
 template <bool TAU>
-__device__ __forceinline__ float rk4_half_z(const TraceArgs &a, const ZP &z0, const ZP &zm, const ZP &z1, float ox,
+__device__ __forceinline__ float rk4_half_z(float sx, float sy, const ZP &z0, const ZP &zm, const ZP &z1, float ox,
                                             float oy, State &y, float &iWc, uint32_t &far, float &em) {
     // the new state is accumulated as y + h/6 (k1 + 2 k2 + 2 k3 + k4) stage
     // by stage, each weight folded into that stage's factor c / W
@@ -355,35 +355,21 @@ __device__ __forceinline__ float rk4_half_z(const TraceArgs &a, const ZP &z0, co
     float4 g;
     float iW = iWc, vf = 0.f, unused, e1, e2, e3, e4;
     far = 0u;
-    rhs_z<true, true>(a, z0, ox, oy, y, g, iW, vf, far, e1);
+    rhs_z<true, true>(sx, sy, z0, ox, oy, y, g, iW, vf, far, e1);
     const float phi = g.w * vf;
     State yn = axpy_r<TAU>(y, h6 * iW, y, g);
     const State s2 = axpy_r<TAU>(y, 0.25f * iW, y, g);
-    rhs_z<false, true>(a, zm, ox, oy, s2, g, iW, unused, far, e2);
+    rhs_z<false, true>(sx, sy, zm, ox, oy, s2, g, iW, unused, far, e2);
     yn = axpy_r<TAU>(yn, h3 * iW, s2, g);
     const State s3 = axpy_r<TAU>(y, 0.25f * iW, s2, g);
-    rhs_z<false, true>(a, zm, ox, oy, s3, g, iW, unused, far, e3);
+    rhs_z<false, true>(sx, sy, zm, ox, oy, s3, g, iW, unused, far, e3);
     yn = axpy_r<TAU>(yn, h3 * iW, s3, g);
     const State s4 = axpy_r<TAU>(y, 0.5f * iW, s3, g);
-    rhs_z<false, true>(a, z1, ox, oy, s4, g, iW, unused, far, e4);
+    rhs_z<false, true>(sx, sy, z1, ox, oy, s4, g, iW, unused, far, e4);
     y = axpy_r<TAU>(yn, h6 * iW, s4, g);
     iWc = iW;
     em = fmaxf(fmaxf(fabsf(e1), fabsf(e2)), fmaxf(fabsf(e3), fabsf(e4)));
     return phi;
-}
-
-// the plane forms z0, D below from a cell's eight nodes
-__device__ __forceinline__ void planes_of(const float4 &c000, const float4 &c100, const float4 &c010, const float4 &c110,
-                                          const float4 &c001, const float4 &c101, const float4 &c011,
-                                          const float4 &c111, ZP &z0, ZP &D) {
-    z0.A = c000;
-    z0.B = f4sub(c100, c000);
-    z0.Cc = f4sub(c010, c000);
-    z0.E = f4sub(f4sub(c110, c010), z0.B);
-    D.A = f4sub(c001, c000);
-    D.B = f4sub(f4sub(c101, c001), z0.B);
-    D.Cc = f4sub(f4sub(c011, c001), z0.Cc);
-    D.E = f4sub(f4sub(f4sub(c111, c011), f4sub(c101, c001)), z0.E);
 }
 
 // The cell as plane forms: z0 on its lower z-plane and D = (upper - lower),
@@ -403,7 +389,16 @@ __device__ __forceinline__ void load_planes(const TraceArgs &A, int ix, int iy, 
     }
     const int64_t plane = (int64_t)A.nx * A.ny;
     const float4 *p = A.field + node_index(A, ix, iy, iz);
-    planes_of(p[0], p[1], p[A.nx], p[A.nx + 1], p[plane], p[plane + 1], p[plane + A.nx], p[plane + A.nx + 1], z0, D);
+    const float4 c000 = p[0], c100 = p[1], c010 = p[A.nx], c110 = p[A.nx + 1];
+    const float4 c001 = p[plane], c101 = p[plane + 1], c011 = p[plane + A.nx], c111 = p[plane + A.nx + 1];
+    z0.A = c000;
+    z0.B = f4sub(c100, c000);
+    z0.Cc = f4sub(c010, c000);
+    z0.E = f4sub(f4sub(c110, c010), z0.B);
+    D.A = f4sub(c001, c000);
+    D.B = f4sub(f4sub(c101, c001), z0.B);
+    D.Cc = f4sub(f4sub(c011, c001), z0.Cc);
+    D.E = f4sub(f4sub(f4sub(c111, c011), f4sub(c101, c001)), z0.E);
 }
 
 // the plane dt above plane z (D = the cell's upper-minus-lower plane form)
@@ -500,6 +495,7 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
     }
     if (k >= K) return good && lateral_inside(a, pxb, pyb, ys) == in0;
     PhaseLedger L;
+    const float sx = a.sx, sy = a.sy;
     // 1 / W seeding each cached step's Newton refinement: the previous step's
     // last stage, or exact after a gathered step (per lane, so that a lane's
     // results never depend on which other lanes of its wave redid a step)
@@ -536,7 +532,7 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
             const ZP z3 = zstep(zh, 0.25f, D);
             const ZP z1 = zstep(z3, 0.25f, D);
             yn = ys;
-            phi = rk4_half_z<TAU>(a, zh, z3, z1, ox, oy, yn, iWc, far, em);
+            phi = rk4_half_z<TAU>(sx, sy, zh, z3, z1, ox, oy, yn, iWc, far, em);
             ok = far <= kInCell && em <= kNewtonTol && inside;
         } else {  // whole cells from the cache
             bool done = false;
@@ -553,7 +549,7 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
                 const ZP zq = zstep(z0, 0.25f, D);
                 const ZP zh = zstep(z0, 0.5f, D);
                 yn = ys;
-                phi = rk4_half_z<TAU>(a, z0, zq, zh, ox, oy, yn, iWc, far, em);
+                phi = rk4_half_z<TAU>(sx, sy, z0, zq, zh, ox, oy, yn, iWc, far, em);
                 ok = far <= kInCell && em <= kNewtonTol && inside;
                 if (__ballot(!ok) != 0) break;  // redo the cell's first step below
                 ys = yn;
@@ -563,7 +559,7 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
                 const ZP z3 = zstep(zh, 0.25f, D);
                 const ZP z1 = zstep(z3, 0.25f, D);
                 yn = ys;
-                phi = rk4_half_z<TAU>(a, zh, z3, z1, ox, oy, yn, iWc, far, em);
+                phi = rk4_half_z<TAU>(sx, sy, zh, z3, z1, ox, oy, yn, iWc, far, em);
                 ok = far <= kInCell && em <= kNewtonTol && inside;
                 if (__ballot(!ok) != 0) break;  // redo the cell's second step below
                 ledger_second(a, pxb, pyb, k, L, ph, phi, true, 0.f, ys, yn);
@@ -606,10 +602,22 @@ __device__ __forceinline__ bool march_m2(const TraceArgs &a, float pxb, float py
 // bound by VALU issue, and all of that is VALU work march_m2 does per cell:
 // 64-bit lane addresses, selects for the lanes outside the grid, compares
 // turned into integers for the ballots, copies on the loop's back edge (405 ->
-// 360 VALU per cell; 1e7 rays: 35.3 -> 32.7 ms through 512^3, 95.9 -> 91.4 ms
-// through 1024^3, where more steps are redone by gathers; 1e5 rays through
-// 128^3: 206 -> 187 us).  The offset (16 or 64 bytes a node) and the row index are exact in 32 bits and in
-// fp32 while nx ny <= 2^24, hence kUniformPlane.
+// 360 VALU per cell; 1e7 rays: 35.3 -> 32.7 ms through 512^3).
+//
+// A ray stays in its column for tens to hundreds of cells, so a cell takes its
+// lower plane's form from the cell before (the upper form there: the same
+// subtractions on the same nodes) and loads only the four nodes of its upper
+// plane, which were asked for a whole cell earlier.  That is half the loads,
+// none of them waited for, and 20 subtractions fewer (337 VALU per cell), for
+// 126 registers: four waves per SIMD instead of five, which the loads ahead
+// more than make up for, most where few waves are there to hide a load.  Trace
+// kernel, five waves and eight loads a cell -> this: 1e7 rays 31.7 -> 29.7 ms
+// (512^3) and 90.8 -> 85.8 ms (1024^3, where more steps are redone by gathers
+// and a redone step's cell is entered anew), 1e5 rays 736 -> 553 us (512^3)
+// and 156 -> 139 us (128^3), 1e3 rays 49.7 -> 42.4 us (48^3).
+//
+// The offset (16 or 64 bytes a node) and the row index are exact in 32 bits and
+// in fp32 while nx ny <= 2^24, hence kUniformPlane.
 constexpr uint32_t kUniformPlane = 1u << 24;
 
 // lane mask -> this lane's condition
@@ -617,25 +625,26 @@ __device__ __forceinline__ bool lane_of(uint64_t m) { return __builtin_amdgcn_in
 __device__ __forceinline__ uint64_t mask_of(bool c) { return __builtin_amdgcn_ballot_w64(c); }
 
 // The cell of the current position: its byte offset in a plane (off, from the
-// row index computed exactly in fp32), the entry point relative to it, and the
-// lanes whose position lies in the grid.  A position outside is clamped to the
-// nearest cell (its step is redone by gathers); kClampBelow keeps the last
-// node in the last cell.
+// row index computed exactly in fp32), its column (ix, iy), the entry point
+// relative to it, and the lanes whose position lies in the grid.  A position
+// outside is clamped to the nearest cell (its step is redone by gathers); cx,
+// cy, the floats below n - 1, keep the last node in the last cell.
 template <bool FORMS>
-__device__ __forceinline__ uint64_t locate_u(const TraceArgs &a, float pxb, float pyb, float cx, float cy, float fnx,
-                                             const State &s, float &ox, float &oy, uint32_t &off) {
-    const float px = fmaf(a.sx, s.qx, pxb), py = fmaf(a.sy, s.qy, pyb);
-    const float ix = floorf(__builtin_amdgcn_fmed3f(px, 0.f, cx)), iy = floorf(__builtin_amdgcn_fmed3f(py, 0.f, cy));
+__device__ __forceinline__ uint64_t locate_u(const TraceArgs &a, float sx, float sy, float pxb, float pyb, float cx, float cy,
+                                             float fnx, const State &s, float &ix, float &iy, float &ox, float &oy,
+                                             uint32_t &off) {
+    const float px = fmaf(sx, s.qx, pxb), py = fmaf(sy, s.qy, pyb);
+    ix = floorf(__builtin_amdgcn_fmed3f(px, 0.f, cx));
+    iy = floorf(__builtin_amdgcn_fmed3f(py, 0.f, cy));
     ox = pxb - ix;
     oy = pyb - iy;
     off = (uint32_t)fmaf(iy, fnx, ix) * (FORMS ? 64u : 16u);
     return mask_of(__float_as_uint(px) <= __float_as_uint(a.fx1)) & mask_of(__float_as_uint(py) <= __float_as_uint(a.fy1));
 }
 
-// load_planes from the address of node (0, 0) of the cell's lower plane, the
-// bytes from row to row and plane to plane, and the lane's offset.  The
-// pointers are to global memory by type: a batch item's come from memory,
-// where the compiler could not tell and would emit flat loads.
+// Loads of the node field by a pointer that is to global memory by type: a
+// batch item's comes from memory, where the compiler could not tell and would
+// emit flat loads.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) char *gbytes;
 __device__ __forceinline__ float4 gload4(gbytes p) {
@@ -643,18 +652,28 @@ __device__ __forceinline__ float4 gload4(gbytes p) {
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
+// The four nodes of one plane of a cell (FORMS: their plane form, as stored),
+// from the address of the plane's node (0, 0), the bytes from row to row and
+// the lane's offset.
+struct Nodes {
+    float4 a, b, c, e;
+};
 template <bool FORMS>
-__device__ __forceinline__ void load_planes_u(gbytes base, int64_t row, int64_t step, uint32_t off, ZP &z0, ZP &D) {
-    const gbytes p0 = base + off, q0 = base + step + off;
-    if (FORMS) {
-        z0 = ZP{gload4(p0), gload4(p0 + 16), gload4(p0 + 32), gload4(p0 + 48)};
-        D = ZP{f4sub(gload4(q0), z0.A), f4sub(gload4(q0 + 16), z0.B), f4sub(gload4(q0 + 32), z0.Cc),
-               f4sub(gload4(q0 + 48), z0.E)};
-        return;
-    }
-    const gbytes p1 = base + row + off, q1 = base + step + row + off;
-    planes_of(gload4(p0), gload4(p0 + 16), gload4(p1), gload4(p1 + 16), gload4(q0), gload4(q0 + 16), gload4(q1),
-              gload4(q1 + 16), z0, D);
+__device__ __forceinline__ Nodes load_nodes(gbytes base, int64_t row, uint32_t off) {
+    const gbytes p = base + off;
+    if (FORMS) return Nodes{gload4(p), gload4(p + 16), gload4(p + 32), gload4(p + 48)};
+    const gbytes q = base + row + off;
+    return Nodes{gload4(p), gload4(p + 16), gload4(q), gload4(q + 16)};
+}
+// their plane form (the subtractions of load_planes, so the same bits)
+template <bool FORMS>
+__device__ __forceinline__ ZP form_of(const Nodes &n) {
+    if (FORMS) return ZP{n.a, n.b, n.c, n.e};
+    const float4 B = f4sub(n.b, n.a);
+    return ZP{n.a, B, f4sub(n.c, n.a), f4sub(f4sub(n.e, n.c), B)};
+}
+__device__ __forceinline__ ZP zsub(const ZP &u, const ZP &z) {
+    return ZP{f4sub(u.A, z.A), f4sub(u.B, z.B), f4sub(u.Cc, z.Cc), f4sub(u.E, z.E)};
 }
 
 template <bool TAU, bool FORMS>
@@ -672,48 +691,72 @@ __device__ __forceinline__ bool march_m2u(const TraceArgs &a, float pxb, float p
         constexpr int NB = FORMS ? 64 : 16;
         const float cx = __uint_as_float(__float_as_uint(a.fx1) - 1u), cy = __uint_as_float(__float_as_uint(a.fy1) - 1u);
         const float fnx = (float)a.nx;
+        // held in vector registers: a v_fma with a scalar register operand issues
+        // at half the rate of one on vector registers
+        float sx = a.sx, sy = a.sy;
+        asm("" : "+v"(sx), "+v"(sy));
         // bytes from plane to plane and row to row
         const int64_t step = (int64_t)a.plane * NB, row = (int64_t)a.nx * NB;
-        gbytes base = (gbytes)(FORMS ? a.forms : a.field) + (k >> 1) * step;
+        const gbytes base0 = (gbytes)(FORMS ? a.forms : a.field);
+        gbytes base = base0 + (k >> 1) * step;
         PhaseLedger L;
         float iWc = __builtin_amdgcn_rcpf(1.0f + ys.Wd);
+        const gbytes last = base0 + (int64_t)(a.nz - 1) * step;
         for (;;) {
-            float ox, oy, phi, em;
+            float ix, iy, ox, oy, phi, em;
             uint32_t off, far;
-            uint64_t in, okm;
+            uint64_t in = locate_u<FORMS>(a, sx, sy, pxb, pyb, cx, cy, fnx, ys, ix, iy, ox, oy, off), okm;
+            crossed |= in ^ in0;
             State yn;
-            // whole cells from the cache
-            for (;;) {
-                ZP z0, D;
-                // raised wave priority while the cell's loads are issued (march_m2)
+            ZP zc = form_of<FORMS>(load_nodes<FORMS>(base, row, off));
+            Nodes up = load_nodes<FORMS>(base + step, row, off);
+            // One whole cell from the cache: its lower plane's form zc comes from
+            // the cell before, the upper one's is left in U for the next; the
+            // nodes above that are loaded a cell ahead.  Returns whether another
+            // cell follows.
+            auto cell = [&](ZP &zc, ZP &U) __attribute__((always_inline)) {
+                U = form_of<FORMS>(up);
+                const ZP D = zsub(U, zc);
+                const ZP zq = zstep(zc, 0.25f, D);
+                const ZP zh = zstep(zc, 0.5f, D);
                 __builtin_amdgcn_s_setprio(1);
-                in = locate_u<FORMS>(a, pxb, pyb, cx, cy, fnx, ys, ox, oy, off);
-                load_planes_u<FORMS>(base, row, step, off, z0, D);
+                const gbytes ahead = base + 2 * step;
+                up = load_nodes<FORMS>(ahead < last ? ahead : last, row, off);
                 __builtin_amdgcn_s_setprio(0);
-                crossed |= in ^ in0;
-                const ZP zq = zstep(z0, 0.25f, D);
-                const ZP zh = zstep(z0, 0.5f, D);
                 yn = ys;
-                phi = rk4_half_z<TAU>(a, z0, zq, zh, ox, oy, yn, iWc, far, em);
+                phi = rk4_half_z<TAU>(sx, sy, zc, zq, zh, ox, oy, yn, iWc, far, em);
                 okm = mask_of(far <= kInCell) & mask_of(em <= kNewtonTol) & in;
-                if (__builtin_expect(okm != act, 0)) break;
+                if (__builtin_expect(okm != act, 0)) return false;
                 ledger_first(L, ph, phi, true, 0.f);
                 good &= mask_of(yn.Wd > kWdMin);
                 ys = yn;
                 ++k;
                 const ZP z3 = zstep(zh, 0.25f, D);
                 const ZP z1 = zstep(z3, 0.25f, D);
-                phi = rk4_half_z<TAU>(a, zh, z3, z1, ox, oy, yn, iWc, far, em);
+                phi = rk4_half_z<TAU>(sx, sy, zh, z3, z1, ox, oy, yn, iWc, far, em);
                 okm = mask_of(far <= kInCell) & mask_of(em <= kNewtonTol) & in;
-                if (__builtin_expect(okm != act, 0)) break;
+                if (__builtin_expect(okm != act, 0)) return false;
                 ledger_smooth(L, ph, phi);
                 good &= mask_of(yn.Wd > kWdMin);
                 ys = yn;
                 ++k;
                 base += step;
-                if (k >= K) break;
+                if (k >= K) return false;
+                // the next cell: in the same column unless a lane has left it
+                const float px = fmaf(sx, ys.qx, pxb), py = fmaf(sy, ys.qy, pyb);
+                const uint32_t ux = __float_as_uint(px - ix), uy = __float_as_uint(py - iy);  // exact
+                if (__builtin_expect(mask_of(max(ux, uy) < kInCell) != act, 0)) {
+                    in = locate_u<FORMS>(a, sx, sy, pxb, pyb, cx, cy, fnx, ys, ix, iy, ox, oy, off);
+                    crossed |= in ^ in0;
+                    U = form_of<FORMS>(load_nodes<FORMS>(base, row, off));
+                    up = load_nodes<FORMS>(base + step, row, off);
+                }
+                return true;
+            };
+            ZP zb;
+            while (cell(zc, zb) && cell(zb, zc)) {  // two cells a turn: no copies from U to zc
             }
-            // the three ways out of that loop meet here: hidden from the compiler,
+            // the ways out of that loop meet here: hidden from the compiler,
             // which would otherwise give each its own copy of what follows and
             // pay for it with register copies on the loop's common path
             asm volatile("" : "+s"(okm), "+s"(k));
@@ -737,20 +780,20 @@ __device__ __forceinline__ bool march_m2u(const TraceArgs &a, float pxb, float p
                 if (!(k & 1)) break;
                 // the cell's second step: the lanes that redid the first one
                 // locate the cell they are in now, the others reload their own
-                float ox2, oy2;
+                float ix2, iy2, ox2, oy2;
                 uint32_t off2;
-                const uint64_t in2 = locate_u<FORMS>(a, pxb, pyb, cx, cy, fnx, ys, ox2, oy2, off2);
+                const uint64_t in2 = locate_u<FORMS>(a, sx, sy, pxb, pyb, cx, cy, fnx, ys, ix2, iy2, ox2, oy2, off2);
                 crossed |= (in2 ^ in0) & ~okm;
                 in = (in & okm) | (in2 & ~okm);
                 ox = ok ? ox : ox2;
                 oy = ok ? oy : oy2;
                 off = ok ? off : off2;
-                ZP u0, uD;
-                load_planes_u<FORMS>(base, row, step, off, u0, uD);
+                const ZP u0 = form_of<FORMS>(load_nodes<FORMS>(base, row, off));
+                const ZP uD = zsub(form_of<FORMS>(load_nodes<FORMS>(base + step, row, off)), u0);
                 const ZP uh = zstep(u0, 0.5f, uD);
                 const ZP u3 = zstep(uh, 0.25f, uD);
                 const ZP u1 = zstep(u3, 0.25f, uD);
-                phi = rk4_half_z<TAU>(a, uh, u3, u1, ox, oy, yn, iWc, far, em);
+                phi = rk4_half_z<TAU>(sx, sy, uh, u3, u1, ox, oy, yn, iWc, far, em);
                 okm = mask_of(far <= kInCell) & mask_of(em <= kNewtonTol) & in;
             }
             base += step;
@@ -913,10 +956,9 @@ __device__ __forceinline__ void trace_ray(const TraceArgs &a, int64_t t) {
     if (a.status) a.status[r] = st;
 }
 
-// The h = 1/2 form fits 96 VGPRs (five waves per SIMD) with one 8-byte spill
-// outside the step loop.
+// The h = 1/2 form takes 126 VGPRs (march_m2u): four waves per SIMD.
 template <bool CACHED, bool M2, bool TAU, bool FORMS = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M2 ? 5 : 1))) void trace_rk4_kernel(TraceArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M2 ? 4 : 1))) void trace_rk4_kernel(TraceArgs a) {
     const int b = tt::xcd_block((int)blockIdx.x, (int)gridDim.x);
     const int64_t t = (int64_t)b * blockDim.x + threadIdx.x;
     if (t >= a.n) return;
@@ -938,7 +980,7 @@ __global__ void reset_kernel(BatchHeader *h) {
 }
 
 template <bool CACHED, bool M2>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M2 ? 5 : 4))) void trace_batch_kernel(BatchHeader *hdr, const TraceArgs *__restrict__ items,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void trace_batch_kernel(BatchHeader *hdr, const TraceArgs *__restrict__ items,
                                                           const int32_t *__restrict__ chunk_item,
                                                           const int64_t *__restrict__ chunk_start, int nchunks,
                                                           int chunk) {
