@@ -432,6 +432,43 @@ int tt_surrogate_loss(const float *Y, int64_t ldy, const float *T, int64_t ldt, 
  * bf16 copy w_bf16 when non-NULL. */
 int tt_adam(float *w, const float *g, float *m, float *v, void *w_bf16, int64_t n, double lr, double b1, double b2,
             double eps, int64_t step, double weight_decay, void *stream);
+/* One training step of the network nfeat -> 256 -> 256 -> 256 -> 8 (GELU on
+ * the hidden layers): forward, tt_surrogate_loss, backward and Adam over the
+ * rows rows[0 .. batch) (device int64) of X (bf16 standardised features, row
+ * stride ldx) and T (fp32 targets, row stride ldt), with the arithmetic of
+ * tt_gemm_bf16 / tt_gelu_backward / tt_adam called layer by layer.  nfeat: a
+ * multiple of 8, at most 64.  Layer l's weights are [out][in]; w_bf16 holds
+ * their bf16 copy and, for l > 0, wt_bf16 its transpose [in][out]; both are
+ * read and refreshed.  dw, db receive the gradients, m*, v* are Adam's
+ * moments.  w_reg, err_lo and err_hi are host values (n_reg + n_err <= 8).
+ * workspace: tt_mlp_train_workspace_bytes(batch) bytes of device memory, one
+ * per stream that steps run on; its contents need not be kept between steps.
+ * The two loss sums are ADDED to loss_out (2 device doubles). */
+typedef struct {
+    float *w, *b;
+    void *w_bf16, *wt_bf16;
+    float *dw, *db, *mw, *vw, *mb, *vb;
+} tt_mlp_layer;
+typedef struct {
+    tt_mlp_layer layer[4];
+    const void *X;
+    int64_t ldx;
+    const float *T;
+    int64_t ldt;
+    const int64_t *rows;
+    int32_t batch, nfeat;
+    int32_t n_reg, n_err;
+    float w_reg[8];
+    int32_t err_lo[4], err_hi[4];
+    double tau;
+    double lr, b1, b2, eps, weight_decay;
+    int64_t step;
+    void *workspace;
+    size_t workspace_bytes;
+    double *loss_out;
+} tt_mlp_train;
+int tt_mlp_train_workspace_bytes(int32_t batch, size_t *bytes);
+int tt_mlp_train_step(const tt_mlp_train *args, void *stream);
 /* out (bf16, [rows][ldo], zero-padded) = (x - mu) * inv_sd over cols, with
  * x element (r, c) at x[r * srow + c * scol] */
 int tt_standardize_bf16(const float *x, int64_t srow, int64_t scol, int64_t rows, int32_t cols, const float *mu,

@@ -63,6 +63,19 @@ class GemmArgs(C.Structure):
                 ("ldc", C.c_int64), ("Zpre", C.c_void_p), ("ksplit", C.c_int32)]
 
 
+class MlpLayer(C.Structure):
+    _fields_ = [(k, C.c_void_p) for k in ("w", "b", "w_bf16", "wt_bf16", "dw", "db", "mw", "vw", "mb", "vb")]
+
+
+class MlpTrain(C.Structure):
+    _fields_ = [("layer", MlpLayer * 4), ("X", C.c_void_p), ("ldx", C.c_int64), ("T", C.c_void_p), ("ldt", C.c_int64),
+                ("rows", C.c_void_p), ("batch", C.c_int32), ("nfeat", C.c_int32), ("n_reg", C.c_int32),
+                ("n_err", C.c_int32), ("w_reg", C.c_float * 8), ("err_lo", C.c_int32 * 4), ("err_hi", C.c_int32 * 4),
+                ("tau", C.c_double), ("lr", C.c_double), ("b1", C.c_double), ("b2", C.c_double), ("eps", C.c_double),
+                ("weight_decay", C.c_double), ("step", C.c_int64), ("workspace", C.c_void_p),
+                ("workspace_bytes", C.c_size_t), ("loss_out", C.c_void_p)]
+
+
 class BatchItem(C.Structure):
     _fields_ = [("field4", C.c_void_p), ("grid", Grid), ("s0", C.c_void_p), ("ld_s0", C.c_int64),
                 ("n", C.c_int64), ("order", C.c_void_p), ("rf", C.c_void_p), ("ld_rf", C.c_int64),
@@ -111,6 +124,8 @@ _SIGNATURES = {
     "tt_bias_grad": [P, I64, I32, I64, P, P],
     "tt_surrogate_loss": [P, I64, P, I64, P, I64, I64, I32, P, I32, P, P, D, I32, P, P],
     "tt_adam": [P, P, P, P, P, I64, D, D, D, D, I64, D, P],
+    "tt_mlp_train_workspace_bytes": [I32, SIZE_P],
+    "tt_mlp_train_step": [C.POINTER(MlpTrain), P],
     "tt_batch_workspace_bytes": [C.POINTER(BatchItem), I32, I32, C.POINTER(C.c_size_t)],
     "tt_batch_prepare": [C.POINTER(BatchItem), I32, D, I32, P, C.c_size_t, C.POINTER(BatchInfo)],
     "tt_batch_trace": [P, C.POINTER(BatchInfo), C.POINTER(BatchTuning), P],

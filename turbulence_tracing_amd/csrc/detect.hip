@@ -99,13 +99,7 @@ constexpr int kDetRays = 4;                       // rays per thread
 constexpr int kDetBlockRays = kDetBlock * kDetRays;
 constexpr int kLdsBins = 8192;  // private window: 32 KB of uint32/float
 
-// LDS-only workgroup barrier: the fences order LDS operations only, so the
-// barrier does not wait for this wave's global atomics to complete
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
+using tt::lds_barrier;
 
 __device__ __forceinline__ int wave_min(int v) {
     for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));

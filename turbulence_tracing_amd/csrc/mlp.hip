@@ -15,6 +15,7 @@
 // split-K the partial tiles are added atomically into fp32 C.
 #include <hip/hip_bf16.h>
 
+#include "gelu.h"
 #include "tt_internal.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -26,21 +27,8 @@ namespace {
 constexpr int BM = 64, BN = 64, BK = 32;
 constexpr int PADK = 8;  // LDS row padding (bf16 elements) to spread banks
 
-// GELU, tanh form: 0.5 x (1 + tanh(u)), u = sqrt(2/pi) (x + 0.044715 x^3),
-// evaluated as x * s with s = 0.5 (1 + tanh(u)) = 1 / (1 + exp(-2u)) and
-// exp(-2u) = 2^(x (a + b x^2)), a = -2 sqrt(2/pi) log2(e), b = 0.044715 a.
-// Saturates correctly: s -> 0 (exp2 -> inf) and s -> 1 (exp2 -> 0).
-__device__ __forceinline__ float gelu_s(float x) {
-    const float e = __builtin_amdgcn_exp2f(x * fmaf(-0.1029432395800235f, x * x, -2.302208198144325f));
-    return __builtin_amdgcn_rcpf(1.0f + e);
-}
-__device__ __forceinline__ float gelu_f(float x) { return x * gelu_s(x); }
-// d/dx [x s(2u)] = s + x 2 s (1 - s) u', u' = sqrt(2/pi) (1 + 3 * 0.044715 x^2)
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float s = gelu_s(x);
-    const float du = 0.7978845608028654f * fmaf(0.134145f, x * x, 1.0f);
-    return fmaf(2.0f * x * s * (1.0f - s), du, s);
-}
+using tt::gelu_f;
+using tt::gelu_grad;
 
 // Fill a [64 rows][32 k] LDS tile of operand X(row, k) = X[row*srow + k*sk].
 // mode 1: contiguous along k (8 consecutive k per thread); mode 2: contiguous
@@ -309,13 +297,7 @@ __device__ __forceinline__ void copy_chunk(const __bf16 *w, int chunk, __bf16 *b
                                              (lds_void *)(dst + i * 256 + wave * 64), 16, 0, 0);
 }
 
-// LDS-only workgroup barrier: the fences order LDS operations only, so the
-// barrier does not wait for this wave's global loads
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
+using tt::lds_barrier;
 
 // The two buffers are separate LDS arrays, so the compiler can tell a copy
 // into one from the reads of the other and does not wait for the copy first.

@@ -87,6 +87,14 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
     return x * q + min(x, r) + b / 8;
 }
 
+// LDS-only workgroup barrier: the fences order LDS operations only, so the
+// barrier does not wait for this wave's global loads, stores and atomics
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // W - 1 (W = vz / c) at or below which the z-march hands a ray over to the
 // time integrator (the rule is stated with the tracer)
 constexpr float kWdMin = -0.03f;

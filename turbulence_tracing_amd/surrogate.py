@@ -358,6 +358,7 @@ class Surrogate:
         """Adam with cosine decay on (features, normalised targets)."""
         N = feat.shape[0]
         X = self.standardize(feat)
+        fused = self._fused_step(X, target, batch, wd)
         gen = torch.Generator(device=self.device).manual_seed(seed)
         steps = epochs * (N // batch)
         loss = torch.zeros(2, dtype=torch.float64, device=self.device)
@@ -370,6 +371,11 @@ class Surrogate:
             loss.zero_()
             for b in range(N // batch):
                 idx = perm[b * batch:(b + 1) * batch]
+                lr_t = lr_min + 0.5 * (lr - lr_min) * (1 + np.cos(np.pi * st / max(1, steps)))
+                st += 1
+                if fused is not None:
+                    fused(idx, lr_t, loss)
+                    continue
                 xb = X.index_select(0, idx)
                 tb = target.index_select(0, idx)
                 self.mlp.forward(xb, out=Y, keep=True)
@@ -377,14 +383,47 @@ class Surrogate:
                                            N_ERR, _p(self.err_lo), _p(self.err_hi), float(self.tau), NOUT,
                                            _p(loss), _lib.stream_ptr())
                 self.mlp.backward(dY)
-                lr_t = lr_min + 0.5 * (lr - lr_min) * (1 + np.cos(np.pi * st / max(1, steps)))
                 self.mlp.adam(lr_t, wd=wd)
-                st += 1
             l = (loss / (N // batch * batch)).cpu().numpy()
             hist.append(l)
             if log:
                 log(f"epoch {ep + 1}/{epochs}: mse {l[0]:.4g}  err-head pinball {l[1]:.4g}")
         return hist
+
+    def _fused_step(self, X, target, batch, wd):
+        """The training step as one library call (tt_mlp_train_step: three
+        launches instead of 45), or None where it does not serve: a network
+        of another shape than the surrogate's, a replaced MLP class, or
+        targets that are not this loss's fp32 columns on the device.  Returns
+        a function of (row indices of the batch, learning rate, loss sums)."""
+        m = self.mlp
+        if (type(m) is not MLP or len(m.dims) != 5 or m.dims[1:4] != (256, 256, 256) or m.dims[4] != NOUT or
+                m.dims[0] != NFEAT or batch < 1 or target.dtype != torch.float32 or target.device != X.device or
+                target.dim() != 2 or target.shape[1] != N_REG or target.shape[0] < X.shape[0]):
+            return None
+        T = target if target.stride(1) == 1 and target.stride(0) >= N_REG else target.contiguous()
+        Wt = [None] + [w.t().contiguous() for w in m.Wb[1:]]
+        nbytes = C.c_size_t()
+        self.lib.tt_mlp_train_workspace_bytes(batch, C.byref(nbytes))
+        ws = torch.empty(nbytes.value, dtype=torch.uint8, device=self.device)
+        a = _lib.MlpTrain()
+        for l in range(4):
+            a.layer[l] = _lib.MlpLayer(*(_p(t) for t in (m.W[l], m.b[l], m.Wb[l], Wt[l], m.dW[l], m.db[l], m.mW[l],
+                                                         m.vW[l], m.mb[l], m.vb[l])))
+        a.X, a.ldx, a.T, a.ldt = _p(X), X.stride(0), _p(T), T.stride(0)
+        a.batch, a.nfeat, a.n_reg, a.n_err = batch, NFEAT, N_REG, N_ERR
+        a.w_reg[:N_REG] = self.w_reg.tolist()
+        a.err_lo[:N_ERR], a.err_hi[:N_ERR] = self.err_lo.tolist(), self.err_hi.tolist()
+        a.tau, a.b1, a.b2, a.eps, a.weight_decay = float(self.tau), 0.9, 0.999, 1e-8, float(wd)
+        a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes.value
+        keep = (X, T, Wt, ws)
+
+        def step(idx, lr, loss, _keep=keep):
+            m.step += 1
+            a.rows, a.lr, a.step, a.loss_out = idx.data_ptr(), float(lr), m.step, loss.data_ptr()
+            self.lib.tt_mlp_train_step(C.byref(a), _lib.stream_ptr())
+
+        return step
 
     def calibrate(self, feat, resid, bar_pos=1e-6, bar_ang=1e-6, margin=0.8, max_scale=1e6):
         """Scale the error heads on held-out rays (features ``feat`` [n, 48]
