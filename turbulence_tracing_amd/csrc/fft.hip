@@ -156,79 +156,14 @@ __device__ __forceinline__ void pass_r_body(float2 *buf, int n, int stride, int 
     __syncthreads();
 }
 
-template <int R>
-__device__ __noinline__ void pass_r(float2 *buf, int n, int stride, int B, int Ns, const float2 *tw) {
-    pass_r_body<R>(buf, n, stride, B, Ns, tw);
-}
-
-// Direct DFT pass for any radix R (odd primes > 5): one output per item.
-__device__ __noinline__ void pass_generic(float2 *buf, int n, int stride, int B, int Ns, int R, const float2 *tw) {
-    float2 o[kElems];
-    const int nbf = n / R;
-    const int total = B * n;
-    const int twstep = n / (Ns * R);
-#pragma unroll
-    for (int i = 0; i < kElems; ++i) {
-        const int g = threadIdx.x + i * kThreads;
-        o[i] = make_float2(0.f, 0.f);
-        if (g < total) {
-            const int p = g / n, e = g - p * n;
-            const int q = e / nbf, b = e - q * nbf;
-            const int k = b % Ns;
-            const float2 *pb = buf + p * stride;
-            float2 acc = make_float2(0.f, 0.f);
-            int qr = 0;  // (q * r) mod R
-            for (int r = 0; r < R; ++r) {
-                float2 x = pb[b + r * nbf];
-                if (k) x = cmul(x, tw[r * k * twstep]);
-                const float2 w = tw[qr * nbf];
-                acc.x += x.x * w.x - x.y * w.y;
-                acc.y += x.x * w.y + x.y * w.x;
-                qr += q;
-                if (qr >= R) qr -= R;
-            }
-            o[i] = acc;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kElems; ++i) {
-        const int g = threadIdx.x + i * kThreads;
-        if (g < total) {
-            const int p = g / n, e = g - p * n;
-            const int q = e / nbf, b = e - q * nbf;
-            const int k = b % Ns;
-            buf[p * stride + (b / Ns) * Ns * R + k + q * Ns] = o[i];
-        }
-    }
-    __syncthreads();
-}
-
-__device__ void lds_fft(float2 *buf, int stride, int B, const AxisPlan &ap, const float2 *tw) {
-    int Ns = 1;
-    for (int s = 0; s < ap.nrad; ++s) {
-        const int R = ap.rad[s];
-        switch (R) {
-            case 8: pass_r<8>(buf, ap.n, stride, B, Ns, tw); break;
-            case 4: pass_r<4>(buf, ap.n, stride, B, Ns, tw); break;
-            case 2: pass_r<2>(buf, ap.n, stride, B, Ns, tw); break;
-            case 3: pass_r<3>(buf, ap.n, stride, B, Ns, tw); break;
-            case 5: pass_r<5>(buf, ap.n, stride, B, Ns, tw); break;
-            default: pass_generic(buf, ap.n, stride, B, Ns, R, tw); break;
-        }
-        Ns *= R;
-    }
-}
-
 // ---------------------------------------------------------------------
 // Fixed lengths (128, 192, 256, 384, 512, 1024: powers of two times at most
 // one 3) with every size known at compile time, so the index arithmetic is shifts and masks, and with the first and
 // the last Stockham pass in registers: the first pass reads its butterfly
 // inputs straight from the pass's loader (global memory or the generator)
 // and the last one hands its outputs straight to the storer, so a pencil
-// goes through LDS twice fewer than with LDS-to-LDS passes only.  Same radix
-// order as factorize (8 while 8 divides what is left, then 4 or 2, then the
-// odd prime).
+// goes through LDS twice fewer than with LDS-to-LDS passes only.  Radices: 8
+// while 8 divides what is left, then 4 or 2, then the odd prime.
 template <int N, int NS>
 constexpr int radix_at() {
     int m = N / NS, e = 0;
@@ -335,7 +270,7 @@ struct PassArgs {
     AxisPlan ap;
     const float2 *tw;  // twiddles of this axis, e^{+2 pi i m / n}
     int nx, ny, nz, nxh;
-    int B;
+    int lb;        // any length: log2 of the pencils per block
     float2 *spec;  // [nz][ny][nxh]
     // native spectrum
     double aniso, kmin, kmax;
@@ -473,120 +408,42 @@ __device__ __forceinline__ void bin_power(const PassArgs &a, int jx, int jy, int
 }
 #pragma clang fp contract(on)
 
-// NF > 0: the pencil length is NF (one of the fixed lengths) and B = kBatch / NF, both
-// compile-time constants; NF == 0: any length, from the plan.
+// add the block's sum of v to *out
+template <int THREADS>
+__device__ __forceinline__ void block_sum(double v, double *out) {
+    __shared__ double red[THREADS / 64];
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < THREADS / 64; ++w) t += red[w];
+        atomicAdd(out, t);
+    }
+}
+
+// The fixed lengths: NF points a pencil, kBatch / NF pencils a block.
 template <int MODE, int NF>
 __global__ __launch_bounds__(kThreads) void fft_pass_kernel(PassArgs a) {
     extern __shared__ float2 smem[];
-    const int n = NF ? NF : a.ap.n;
-    const int stride = n + 1;
-    const int B = NF ? kBatch / NF : a.B;
+    constexpr int BF = kBatch / NF;
     float2 *buf = smem;
-    float2 *tw = smem + B * stride;
-    for (int j = threadIdx.x; j < n; j += kThreads) tw[j] = a.tw[j];
-    const int total = B * n;
-
-    if constexpr (NF > 0) {
-        constexpr int BF = kBatch / NF;
-        if constexpr (MODE == kPowZ) {
-            double *hs = reinterpret_cast<double *>(tw + NF), *hc = hs + a.nbins;
-            for (int j = threadIdx.x; j < 2 * a.nbins; j += kThreads) hs[j] = 0.0;
-            const int kx0 = blockIdx.x * BF, fixed = blockIdx.y;
-            fft_pow2<NF, true>(
-                buf, tw,
-                [&](int p, int j) {
-                    const int kx = kx0 + p;
-                    return kx < a.nxh ? a.spec[((int64_t)j * a.ny + fixed) * a.nxh + kx] : make_float2(0.f, 0.f);
-                },
-                [&](int p, int j, float2 v) {
-                    const int kx = kx0 + p;
-                    if (kx < a.nxh) bin_power(a, kx, fixed, j, v.x * v.x + v.y * v.y, hs, hc);
-                });
-            __syncthreads();
-            for (int j = threadIdx.x; j < a.nbins; j += kThreads) {
-                if (hc[j] != 0.0) {
-                    atomicAdd(&a.hsum[j], hs[j]);
-                    atomicAdd(&a.hcnt[j], hc[j]);
-                }
-            }
-        } else if constexpr (MODE == kFwdX) {
-            const int64_t rows = (int64_t)a.ny * a.nz, r0 = (int64_t)blockIdx.x * BF;
-            fft_pow2<NF, false>(
-                buf, tw,
-                [&](int p, int k) { return make_float2(r0 + p < rows ? a.in[(r0 + p) * NF + k] : 0.f, 0.f); },
-                [&](int p, int k, float2 v) {
-                    if (r0 + p < rows && k < a.nxh) a.spec[(r0 + p) * a.nxh + k] = v;
-                });
-        } else if constexpr (MODE == kPassX) {
-            const int64_t rows = (int64_t)a.ny * a.nz, r0 = (int64_t)blockIdx.x * BF;
-            double ss = 0.0;
-            fft_pow2<NF, false>(
-                buf, tw,
-                [&](int p, int k) {
-                    if (r0 + p >= rows) return make_float2(0.f, 0.f);
-                    const float2 *srow = a.spec + (r0 + p) * a.nxh;
-                    if (k < a.nxh) return srow[k];
-                    const float2 c = srow[NF - k];
-                    return make_float2(c.x, -c.y);
-                },
-                [&](int p, int k, float2 v) {
-                    if (r0 + p >= rows) return;
-                    const float o = v.x * a.scale;
-                    a.out[(r0 + p) * NF + k] = o;
-                    ss += (double)o * (double)o;
-                });
-            if (a.sumsq) {
-                __shared__ double red[kThreads / 64];
-                for (int off = 32; off > 0; off >>= 1) ss += __shfl_down(ss, off, 64);
-                if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-                __syncthreads();
-                if (threadIdx.x == 0) {
-                    double t = 0.0;
-                    for (int w = 0; w < kThreads / 64; ++w) t += red[w];
-                    atomicAdd(a.sumsq, t);
-                }
-            }
-        } else {  // kGenNative, kGenNoise (pencils along z) and kPassY (along y)
-            const int kx0 = blockIdx.x * BF, fixed = blockIdx.y;
-            fft_pow2<NF, true>(
-                buf, tw,
-                [&](int p, int j) {
-                    const int kx = kx0 + p;
-                    if (kx >= a.nxh) return make_float2(0.f, 0.f);
-                    if constexpr (MODE == kPassY)
-                        return a.spec[((int64_t)fixed * a.ny + j) * a.nxh + kx];
-                    else
-                        return gen<MODE>(a, kx, fixed, j);
-                },
-                [&](int p, int j, float2 v) {
-                    const int kx = kx0 + p;
-                    if (kx >= a.nxh) return;
-                    const int64_t idx = (MODE == kPassY) ? ((int64_t)fixed * a.ny + j) * a.nxh + kx
-                                                         : ((int64_t)j * a.ny + fixed) * a.nxh + kx;
-                    a.spec[idx] = v;
-                });
-        }
-    } else if (MODE == kPowZ) {
-        // pencils along z of the half spectrum, then |F|^2 into a block-private
-        // histogram (after the FFT's LDS) flushed with global atomics
-        double *hs = reinterpret_cast<double *>(tw + n), *hc = hs + a.nbins;
+    float2 *tw = smem + BF * (NF + 1);
+    for (int j = threadIdx.x; j < NF; j += kThreads) tw[j] = a.tw[j];
+    if constexpr (MODE == kPowZ) {
+        double *hs = reinterpret_cast<double *>(tw + NF), *hc = hs + a.nbins;
         for (int j = threadIdx.x; j < 2 * a.nbins; j += kThreads) hs[j] = 0.0;
-        const int kx0 = blockIdx.x * B;
-        const int fixed = blockIdx.y;
-        for (int g = threadIdx.x; g < total; g += kThreads) {
-            const int p = g % B, j = g / B;
-            const int kx = kx0 + p;
-            buf[p * stride + j] = kx < a.nxh ? a.spec[((int64_t)j * a.ny + fixed) * a.nxh + kx] : make_float2(0.f, 0.f);
-        }
-        __syncthreads();
-        lds_fft(buf, stride, B, a.ap, tw);
-        for (int g = threadIdx.x; g < total; g += kThreads) {
-            const int p = g % B, j = g / B;
-            const int kx = kx0 + p;
-            if (kx >= a.nxh) continue;
-            const float2 v = buf[p * stride + j];
-            bin_power(a, kx, fixed, j, v.x * v.x + v.y * v.y, hs, hc);
-        }
+        const int kx0 = blockIdx.x * BF, fixed = blockIdx.y;
+        fft_pow2<NF, true>(
+            buf, tw,
+            [&](int p, int j) {
+                const int kx = kx0 + p;
+                return kx < a.nxh ? a.spec[((int64_t)j * a.ny + fixed) * a.nxh + kx] : make_float2(0.f, 0.f);
+            },
+            [&](int p, int j, float2 v) {
+                const int kx = kx0 + p;
+                if (kx < a.nxh) bin_power(a, kx, fixed, j, v.x * v.x + v.y * v.y, hs, hc);
+            });
         __syncthreads();
         for (int j = threadIdx.x; j < a.nbins; j += kThreads) {
             if (hc[j] != 0.0) {
@@ -594,93 +451,305 @@ __global__ __launch_bounds__(kThreads) void fft_pass_kernel(PassArgs a) {
                 atomicAdd(&a.hcnt[j], hc[j]);
             }
         }
-    } else if (MODE == kFwdX) {
-        // real rows along x' -> first nx'/2 + 1 outputs of their transform
-        const int64_t rows = (int64_t)a.ny * a.nz;
-        const int64_t r0 = (int64_t)blockIdx.x * B;
-        for (int g = threadIdx.x; g < total; g += kThreads) {
-            const int p = g / n, k = g - p * n;
-            const int64_t row = r0 + p;
-            buf[p * stride + k] = make_float2(row < rows ? a.in[row * n + k] : 0.f, 0.f);
-        }
-        __syncthreads();
-        lds_fft(buf, stride, B, a.ap, tw);
-        for (int g = threadIdx.x; g < total; g += kThreads) {
-            const int p = g / n, k = g - p * n;
-            const int64_t row = r0 + p;
-            if (row < rows && k < a.nxh) a.spec[row * a.nxh + k] = buf[p * stride + k];
-        }
-    } else if (MODE == kGenNative || MODE == kGenNoise || MODE == kPassY) {
-        // pencils along z (gen) or y: B consecutive kx columns at fixed ky (gen) / z (Y)
-        const int kx0 = blockIdx.x * B;
-        const int fixed = blockIdx.y;
-        for (int g = threadIdx.x; g < total; g += kThreads) {
-            const int p = g % B, j = g / B;
-            const int kx = kx0 + p;
-            float2 v = make_float2(0.f, 0.f);
-            if (kx < a.nxh) {
-                if (MODE == kPassY)
-                    v = a.spec[((int64_t)fixed * a.ny + j) * a.nxh + kx];
-                else
-                    v = gen<MODE>(a, kx, fixed, j);
-            }
-            buf[p * stride + j] = v;
-        }
-        __syncthreads();
-        lds_fft(buf, stride, B, a.ap, tw);
-        for (int g = threadIdx.x; g < total; g += kThreads) {
-            const int p = g % B, j = g / B;
-            const int kx = kx0 + p;
-            if (kx >= a.nxh) continue;
-            const int64_t idx = (MODE == kPassY) ? ((int64_t)fixed * a.ny + j) * a.nxh + kx
-                                                 : ((int64_t)j * a.ny + fixed) * a.nxh + kx;
-            a.spec[idx] = buf[p * stride + j];
-        }
-    } else {
-        // rows along x: complete by Hermitian symmetry, transform, keep Re
-        const int64_t rows = (int64_t)a.ny * a.nz;
-        const int64_t r0 = (int64_t)blockIdx.x * B;
-        for (int g = threadIdx.x; g < total; g += kThreads) {
-            const int p = g / n, k = g - p * n;
-            const int64_t row = r0 + p;
-            float2 v = make_float2(0.f, 0.f);
-            if (row < rows) {
-                const float2 *srow = a.spec + row * a.nxh;
-                if (k < a.nxh) {
-                    v = srow[k];
-                } else {
-                    const float2 c = srow[n - k];
-                    v = make_float2(c.x, -c.y);
-                }
-            }
-            buf[p * stride + k] = v;
-        }
-        __syncthreads();
-        lds_fft(buf, stride, B, a.ap, tw);
+    } else if constexpr (MODE == kFwdX) {
+        const int64_t rows = (int64_t)a.ny * a.nz, r0 = (int64_t)blockIdx.x * BF;
+        fft_pow2<NF, false>(
+            buf, tw,
+            [&](int p, int k) { return make_float2(r0 + p < rows ? a.in[(r0 + p) * NF + k] : 0.f, 0.f); },
+            [&](int p, int k, float2 v) {
+                if (r0 + p < rows && k < a.nxh) a.spec[(r0 + p) * a.nxh + k] = v;
+            });
+    } else if constexpr (MODE == kPassX) {
+        const int64_t rows = (int64_t)a.ny * a.nz, r0 = (int64_t)blockIdx.x * BF;
         double ss = 0.0;
-        for (int g = threadIdx.x; g < total; g += kThreads) {
-            const int p = g / n, k = g - p * n;
-            const int64_t row = r0 + p;
-            if (row >= rows) continue;
-            const float v = buf[p * stride + k].x * a.scale;
-            a.out[row * n + k] = v;
-            ss += (double)v * (double)v;
-        }
-        if (a.sumsq) {
-            // block reduction of the sum of squares
-            __shared__ double red[kThreads / 64];
-            for (int off = 32; off > 0; off >>= 1) ss += __shfl_down(ss, off, 64);
-            if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                double t = 0.0;
-                for (int w = 0; w < kThreads / 64; ++w) t += red[w];
-                atomicAdd(a.sumsq, t);
-            }
-        }
+        fft_pow2<NF, false>(
+            buf, tw,
+            [&](int p, int k) {
+                if (r0 + p >= rows) return make_float2(0.f, 0.f);
+                const float2 *srow = a.spec + (r0 + p) * a.nxh;
+                if (k < a.nxh) return srow[k];
+                const float2 c = srow[NF - k];
+                return make_float2(c.x, -c.y);
+            },
+            [&](int p, int k, float2 v) {
+                if (r0 + p >= rows) return;
+                const float o = v.x * a.scale;
+                a.out[(r0 + p) * NF + k] = o;
+                ss += (double)o * (double)o;
+            });
+        if (a.sumsq) block_sum<kThreads>(ss, a.sumsq);
+    } else {  // kGenNative, kGenNoise (pencils along z) and kPassY (along y)
+        const int kx0 = blockIdx.x * BF, fixed = blockIdx.y;
+        fft_pow2<NF, true>(
+            buf, tw,
+            [&](int p, int j) {
+                const int kx = kx0 + p;
+                if (kx >= a.nxh) return make_float2(0.f, 0.f);
+                if constexpr (MODE == kPassY)
+                    return a.spec[((int64_t)fixed * a.ny + j) * a.nxh + kx];
+                else
+                    return gen<MODE>(a, kx, fixed, j);
+            },
+            [&](int p, int j, float2 v) {
+                const int kx = kx0 + p;
+                if (kx >= a.nxh) return;
+                const int64_t idx = (MODE == kPassY) ? ((int64_t)fixed * a.ny + j) * a.nxh + kx
+                                                     : ((int64_t)j * a.ny + fixed) * a.nxh + kx;
+                a.spec[idx] = v;
+            });
     }
 }
 
+// ---------------------------------------------------------------------
+// Any other length.  A block takes PB pencils (a power of two, 16 up to 600
+// points) in LDS as [element][pencil], two copies of them, and each Stockham
+// pass goes from one to the other: one barrier a pass, and any number of
+// butterflies a thread.  Lanes run over pencils first, so neighbouring lanes
+// share a butterfly: its twiddles are LDS broadcasts, and the columns of passes
+// Y and Z are read and written 128 bytes at a time.  Pencils are numbered
+// through the whole spectrum (not per plane), so only the last block is ragged.
+// The pencil index is XORed with the element's low bits but the last, so that
+// reading along a pencil (pass X loads and stores rows) meets different banks
+// too and two neighbouring pencils stay one aligned 16-byte read.
+// Quotients of small integers are taken in fp32 (exact below 2^21).
+//
+// A prime factor R > 5 is a DFT of R points by definition.  A thread computes
+// kQ consecutive outputs of kP pencils: a term's inputs are read once for kQ
+// outputs and its factors e^{2 pi i q r / R} (from the twiddle table, at q r mod
+// R) once for kP pencils, so (with kQ = 4) 8 complex products go with 5 LDS
+// reads.  The terms are added in order of r: the same bits as one output per
+// thread with two reads a term, as which it was bound by LDS (201^3 = 3 x 67:
+// 1610 us, here 320; 257^3 5700, here 1730); now it is bound by the products'
+// issue.  (With the inputs folded by the symmetry of the factors, on
+// v_mfma_f32_16x16x4_f32, they took 162 and 492 us, but sums in that order move
+// the field's rounding: its sum of squares by more than 1e-9.)  Lengths without
+// such a factor gain from the rest: 300^3 630 -> 330 us, 64^3 87 -> 22 us.
+// 512 threads a block: with 256, 300^3 took 457 us.  Six waves a SIMD: left to
+// itself the compiler takes more registers and 201^3 took 350.
+constexpr int kAnyThreads = 512;
+__device__ __forceinline__ int fdiv(int v, float inv) { return (int)(((float)v + 0.5f) * inv); }
+__device__ __forceinline__ int at(int j, int p, int lb) { return (j << lb) + (p ^ (j & (((1 << lb) - 1) & ~1))); }
+
+template <int R>
+__device__ __forceinline__ void any_pass(const float2 *in, float2 *out, int n, int lb, int Ns, const float2 *tw) {
+    const int nbf = n / R, twstep = nbf / Ns;
+    const float iNs = 1.0f / (float)Ns;
+    const int p = threadIdx.x & ((1 << lb) - 1);
+    for (int b = threadIdx.x >> lb; b < nbf; b += kAnyThreads >> lb) {
+        const int hi = fdiv(b, iNs), k = b - hi * Ns;
+        float2 v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = in[at(b + r * nbf, p, lb)];
+        if (k) {
+#pragma unroll
+            for (int r = 1; r < R; ++r) v[r] = cmul(v[r], tw[r * k * twstep]);
+        }
+        dft<R>(v);
+        const int o = hi * Ns * R + k;
+#pragma unroll
+        for (int q = 0; q < R; ++q) out[at(o + q * Ns, p, lb)] = v[q];
+    }
+}
+
+constexpr int kP = 2;
+
+template <int kQ>
+__device__ __forceinline__ void any_pass_prime(const float2 *in, float2 *out, int n, int lb, int Ns, int R,
+                                               const float2 *tw) {
+    const int nbf = n / R, twstep = nbf / Ns, lg = lb > 1 ? lb - 1 : 0;  // log2 of the pencil groups
+    const int tiles = (R + kQ - 1) / kQ, items = (tiles * nbf) << lg;
+    const float inbf = 1.0f / (float)nbf, iNs = 1.0f / (float)Ns;
+    // byte offsets: a table entry, a row of pencils
+    const uint32_t wrap = (uint32_t)n * 8u, row = (uint32_t)nbf << (lb + 3), swz = lb > 0 ? ((1u << lb) - 2u) * 8u : 0u;
+    const char *tw0 = reinterpret_cast<const char *>(tw), *in0 = reinterpret_cast<const char *>(in);
+    for (int item = threadIdx.x; item < items; item += kAnyThreads) {
+        const int grp = item & ((1 << lg) - 1), bq = item >> lg;
+        const int qt = fdiv(bq, inbf), b = bq - qt * nbf;
+        const int hi = fdiv(b, iNs), k = b - hi * Ns;
+        const int p0 = grp * kP;
+        float2 acc[kQ][kP];
+        uint32_t w[kQ], dw[kQ];  // of entry (q r mod R) nbf, and its step
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+            const int q = min(kQ * qt + j, R - 1);  // spare outputs repeat the last
+            w[j] = 0u;
+            dw[j] = (uint32_t)(q * nbf) * 8u;
+#pragma unroll
+            for (int i = 0; i < kP; ++i) acc[j][i] = make_float2(0.f, 0.f);
+        }
+        uint32_t e8 = (uint32_t)b * 8u, erow = (uint32_t)b << (lb + 3);  // of element b + r nbf
+        for (int r = 0; r < R; ++r, e8 += (uint32_t)nbf * 8u, erow += row) {
+            float2 x[kP];  // at()
+            const char *px = in0 + erow + (((uint32_t)p0 * 8u) ^ (e8 & swz));
+            if (lb > 0) {
+                const float4 xx = *reinterpret_cast<const float4 *>(px);
+                x[0] = make_float2(xx.x, xx.y);
+                x[1] = make_float2(xx.z, xx.w);
+            } else {
+                x[0] = x[1] = *reinterpret_cast<const float2 *>(px);
+            }
+            if (k) {
+                const float2 t = tw[r * k * twstep];
+#pragma unroll
+                for (int i = 0; i < kP; ++i)
+                    x[i] = make_float2(fmaf(x[i].x, t.x, -(x[i].y * t.y)), fmaf(x[i].y, t.x, x[i].x * t.y));
+            }
+#pragma unroll
+            for (int j = 0; j < kQ; ++j) {
+                const float2 c = *reinterpret_cast<const float2 *>(tw0 + w[j]);
+#pragma unroll
+                for (int i = 0; i < kP; ++i) {
+                    // spelled out, so that every build rounds alike
+                    acc[j][i].x = __fadd_rn(acc[j][i].x, fmaf(x[i].x, c.x, -(x[i].y * c.y)));
+                    acc[j][i].y = __fadd_rn(acc[j][i].y, fmaf(x[i].y, c.x, x[i].x * c.y));
+                }
+                w[j] += dw[j];
+                w[j] = min(w[j], w[j] - wrap);  // mod n: the difference wraps to a large value below n
+            }
+        }
+        const int o = hi * Ns * R + k;
+#pragma unroll
+        for (int j = 0; j < kQ; ++j)
+#pragma unroll
+            for (int i = 0; i < kP; ++i)
+                if (kQ * qt + j < R && i < (1 << lb)) out[at(o + (kQ * qt + j) * Ns, p0 + i, lb)] = acc[j][i];
+    }
+}
+
+// The outputs per thread, 2 to 6, for which the block's turns over its items
+// times the work of a turn (as measured, about kQ + 1) are least: 257 points
+// take 520 items of four outputs, so two turns of 512 threads, but 416 of five.
+__device__ __forceinline__ int outputs_per_thread(int R, int nbf, int lb) {
+    int best = 4, least = 1 << 30;
+    for (int q = 2; q <= 6; ++q) {
+        const int items = ((R + q - 1) / q * nbf) << (lb > 1 ? lb - 1 : 0);
+        const int cost = (items + kAnyThreads - 1) / kAnyThreads * (q + 1);
+        if (cost < least) {
+            least = cost;
+            best = q;
+        }
+    }
+    return best;
+}
+
+template <int MODE>
+__global__ __launch_bounds__(kAnyThreads) __attribute__((amdgpu_waves_per_eu(6, 6))) void fft_any_kernel(PassArgs a) {
+    extern __shared__ float2 smem[];
+    const int n = a.ap.n, lb = a.lb, PB = 1 << lb;
+    float2 *buf = smem, *alt = smem + n * PB, *tw = alt + n * PB;
+    double *hs = reinterpret_cast<double *>(tw + n), *hc = hs + a.nbins;
+    for (int j = threadIdx.x; j < n; j += kAnyThreads) tw[j] = a.tw[j];
+    if (MODE == kPowZ)
+        for (int j = threadIdx.x; j < 2 * a.nbins; j += kAnyThreads) hs[j] = 0.0;
+    // pencils: columns (elements `step` apart from `base`) or rows
+    constexpr bool kRows = MODE == kPassX || MODE == kFwdX;
+    const int64_t first = (int64_t)blockIdx.x * PB;
+    const int64_t plane = (int64_t)a.nxh * a.ny;
+    const int p0 = threadIdx.x & (PB - 1), j0 = threadIdx.x >> lb, dj = kAnyThreads >> lb;
+    const int64_t count = kRows ? (int64_t)a.ny * a.nz : MODE == kPassY ? (int64_t)a.nxh * a.nz : plane;
+    const float in_ = 1.0f / (float)n;
+    int kx = 0, ky = 0;
+    int64_t base = 0, step = 0;
+    const bool live = first + p0 < count;
+    if (!kRows) {
+        const uint32_t q = live ? (uint32_t)(first + p0) : 0u;
+        const uint32_t row = q / (uint32_t)a.nxh;
+        kx = (int)(q - row * (uint32_t)a.nxh);
+        ky = (int)row;
+        step = MODE == kPassY ? a.nxh : plane;
+        base = MODE == kPassY ? (int64_t)row * plane + kx : (int64_t)q;
+        for (int j = j0; j < n; j += dj) {
+            float2 v = make_float2(0.f, 0.f);
+            if (live) {
+                if constexpr (MODE == kGenNative || MODE == kGenNoise)
+                    v = gen<MODE>(a, kx, ky, j);
+                else
+                    v = a.spec[base + j * step];
+            }
+            buf[at(j, p0, lb)] = v;
+        }
+    } else {
+        for (int e = threadIdx.x; e < n * PB; e += kAnyThreads) {
+            const int p = fdiv(e, in_), k = e - p * n;
+            const int64_t row = first + p;
+            float2 v = make_float2(0.f, 0.f);
+            if (row < count) {
+                if constexpr (MODE == kFwdX) {
+                    v.x = a.in[row * n + k];
+                } else {  // complete the row by Hermitian symmetry
+                    const bool mirror = k >= a.nxh;
+                    v = a.spec[row * a.nxh + (mirror ? n - k : k)];
+                    if (mirror) v.y = -v.y;
+                }
+            }
+            buf[at(k, p, lb)] = v;
+        }
+    }
+    __syncthreads();
+    int Ns = 1;
+    for (int s = 0; s < a.ap.nrad; ++s) {
+        const int R = a.ap.rad[s];
+        switch (R) {
+            case 8: any_pass<8>(buf, alt, n, lb, Ns, tw); break;
+            case 4: any_pass<4>(buf, alt, n, lb, Ns, tw); break;
+            case 2: any_pass<2>(buf, alt, n, lb, Ns, tw); break;
+            case 3: any_pass<3>(buf, alt, n, lb, Ns, tw); break;
+            case 5: any_pass<5>(buf, alt, n, lb, Ns, tw); break;
+            default:
+                switch (outputs_per_thread(R, n / R, lb)) {
+                    case 2: any_pass_prime<2>(buf, alt, n, lb, Ns, R, tw); break;
+                    case 3: any_pass_prime<3>(buf, alt, n, lb, Ns, R, tw); break;
+                    case 4: any_pass_prime<4>(buf, alt, n, lb, Ns, R, tw); break;
+                    case 5: any_pass_prime<5>(buf, alt, n, lb, Ns, R, tw); break;
+                    default: any_pass_prime<6>(buf, alt, n, lb, Ns, R, tw); break;
+                }
+                break;
+        }
+        Ns *= R;
+        __syncthreads();
+        float2 *t = buf;
+        buf = alt;
+        alt = t;
+    }
+    if constexpr (kRows) {
+        double ss = 0.0;
+        const int w = MODE == kFwdX ? a.nxh : n;  // elements kept of a row
+        const float iw = 1.0f / (float)w;
+        for (int e = threadIdx.x; e < w * PB; e += kAnyThreads) {
+            const int p = fdiv(e, iw), k = e - p * w;
+            const int64_t row = first + p;
+            if (row >= count) continue;
+            const float2 v = buf[at(k, p, lb)];
+            if constexpr (MODE == kFwdX) {
+                a.spec[row * a.nxh + k] = v;
+            } else {
+                const float o = v.x * a.scale;
+                a.out[row * n + k] = o;
+                ss += (double)o * (double)o;
+            }
+        }
+        if (MODE == kPassX && a.sumsq) block_sum<kAnyThreads>(ss, a.sumsq);
+    } else if constexpr (MODE == kPowZ) {
+        if (live)
+            for (int j = j0; j < n; j += dj) {
+                const float2 v = buf[at(j, p0, lb)];
+                bin_power(a, kx, ky, j, v.x * v.x + v.y * v.y, hs, hc);
+            }
+        __syncthreads();
+        for (int j = threadIdx.x; j < a.nbins; j += kAnyThreads) {
+            if (hc[j] != 0.0) {
+                atomicAdd(&a.hsum[j], hs[j]);
+                atomicAdd(&a.hcnt[j], hc[j]);
+            }
+        }
+    } else if (live) {
+        for (int j = j0; j < n; j += dj) a.spec[base + j * step] = buf[at(j, p0, lb)];
+    }
+}
+
+bool fixed_length(int n) { return n == 128 || n == 192 || n == 256 || n == 384 || n == 512 || n == 1024; }
+
+// the passes of a length: 8, then 4 or 2, then the odd primes from the smallest
 void factorize(int n, AxisPlan &ap) {
     ap.n = n;
     ap.nrad = 0;
@@ -704,12 +773,21 @@ void factorize(int n, AxisPlan &ap) {
     }
 }
 
-int pencils_per_block(int n) {
-    int B = kBatch / n;
-    return B < 1 ? 1 : B;
+// LDS of a block: of a fixed length, kBatch / n pencils (padded rows) and the
+// twiddles; of any other, two copies of 2^lb pencils and the twiddles
+constexpr size_t kMaxLds = 160 * 1024 - 256;  // of 160 KB, some static
+size_t smem_fixed(int n) { return ((size_t)kBatch / n * (n + 1) + n) * sizeof(float2); }
+size_t smem_any(int n, int lb) { return (((size_t)2 << lb) + 1) * n * sizeof(float2); }
+// log2 of the pencils a block takes: 16 while two blocks fit a CU's LDS (up to
+// 309 points), then 8, 4 and 2.  One block of 16 alone on a CU leaves it idle
+// between its passes: 640^3 took 8360 us with 8 pencils against 4350 with 4 (256
+// threads), 320^3 816 with 16 against 465 with 8.
+int pencils_any(int n, size_t extra) {
+    int lb = 4;
+    while (lb > 1 && smem_any(n, lb) + extra > kMaxLds / 2) --lb;
+    while (lb > 0 && smem_any(n, lb) + extra > kMaxLds) --lb;
+    return lb;
 }
-
-size_t smem_bytes(int n, int B) { return ((size_t)B * (n + 1) + n) * sizeof(float2); }
 
 }  // namespace
 
@@ -724,7 +802,6 @@ extern "C" int tt_fft_plan_create(int32_t nx, int32_t ny, int32_t nz, tt_fft_pla
     TT_REQUIRE(plan, "tt_fft_plan_create: null plan pointer");
     TT_REQUIRE(nx >= 2 && ny >= 2 && nz >= 2 && nx <= 4096 && ny <= 4096 && nz <= 4096,
                "tt_fft_plan_create: sizes must be in [2, 4096], got %d x %d x %d", nx, ny, nz);
-    TT_REQUIRE(nx <= kBatch && ny <= 65535 && nz <= 65535, "tt_fft_plan_create: size too large");
     tt_fft_plan_s *p = new tt_fft_plan_s();
     p->nx = nx;
     p->ny = ny;
@@ -777,41 +854,61 @@ extern "C" int tt_fft_workspace_bytes(tt_fft_plan plan, size_t *bytes) {
 
 namespace {
 
-#define KERNELS_OF(M)                                                                                   \
-    (const void *)fft_pass_kernel<M, 0>, (const void *)fft_pass_kernel<M, 128>,                         \
-        (const void *)fft_pass_kernel<M, 192>, (const void *)fft_pass_kernel<M, 256>,                   \
-        (const void *)fft_pass_kernel<M, 384>, (const void *)fft_pass_kernel<M, 512>,                   \
-        (const void *)fft_pass_kernel<M, 1024>
-
 // dynamic LDS above 64 KB must be enabled per kernel
 int enable_lds() {
     static int rc = -1;
     if (rc >= 0) return rc;
-    // the largest request: n = 4096 (2 pencils per block), rounded up to 1 KB
-    // (98 KB + 32 KB of power-spectrum bins, within the 160 KB of a CU)
-    const int want = (int)((smem_bytes(4096, pencils_per_block(4096)) + 2 * kMaxBins * sizeof(double) + 1023) /
-                           1024 * 1024);
-    const void *ks[] = {KERNELS_OF(kGenNative), KERNELS_OF(kGenNoise), KERNELS_OF(kPassY),
-                        KERNELS_OF(kPassX),     KERNELS_OF(kFwdX),     KERNELS_OF(kPowZ)};
-    for (const void *k : ks) {
+    const void *any[] = {(const void *)fft_any_kernel<kGenNative>, (const void *)fft_any_kernel<kGenNoise>,
+                         (const void *)fft_any_kernel<kPassY>,     (const void *)fft_any_kernel<kPassX>,
+                         (const void *)fft_any_kernel<kFwdX>,      (const void *)fft_any_kernel<kPowZ>};
+    for (const void *k : any) {
+        hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
+        if (e != hipSuccess) return rc = tt::hip_check(e, "hipFuncSetAttribute(max dynamic LDS)");
+    }
+#define FIXED(M)                                                                                              \
+    (const void *)fft_pass_kernel<M, 128>, (const void *)fft_pass_kernel<M, 192>,                             \
+        (const void *)fft_pass_kernel<M, 256>, (const void *)fft_pass_kernel<M, 384>,                         \
+        (const void *)fft_pass_kernel<M, 512>, (const void *)fft_pass_kernel<M, 1024>
+    const void *fixed[] = {FIXED(kGenNative), FIXED(kGenNoise), FIXED(kPassY),
+                           FIXED(kPassX),     FIXED(kFwdX),     FIXED(kPowZ)};
+#undef FIXED
+    const int want = (int)(smem_fixed(1024) + 2 * kMaxBins * sizeof(double));
+    for (const void *k : fixed) {
         hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, want);
         if (e != hipSuccess) return rc = tt::hip_check(e, "hipFuncSetAttribute(max dynamic LDS)");
     }
     return rc = TT_OK;
 }
 
-// one pass over pencils of length n: the fixed-length kernel for 128, 192,
-// 256, 384, 512 and 1024, the general one otherwise
+// one pass along axis ax (0 x, 1 y, 2 z) of the plan: the fixed-length kernel
+// for 128, 192, 256, 384, 512 and 1024, the one for any length otherwise.
+// extra: LDS behind the FFT's (power-spectrum bins)
 template <int MODE>
-void launch_pass(int n, dim3 grid, size_t sm, hipStream_t st, const PassArgs &a) {
+void launch_pass(tt_fft_plan plan, int ax, hipStream_t st, PassArgs a, size_t extra = 0) {
+    const int n = plan->ax[ax].n;
+    a.ap = plan->ax[ax];
+    a.tw = plan->tw[ax];
+    constexpr bool kRows = MODE == kPassX || MODE == kFwdX;
+    const int64_t rows = (int64_t)plan->ny * plan->nz;
+    if (!fixed_length(n)) {
+        a.lb = pencils_any(n, extra);
+        const int64_t count = kRows ? rows : (int64_t)plan->nxh * (MODE == kPassY ? plan->nz : plan->ny);
+        hipLaunchKernelGGL(fft_any_kernel<MODE>, dim3((unsigned)tt::ceil_div(count, (int64_t)1 << a.lb)),
+                           dim3(kAnyThreads),
+                           smem_any(n, a.lb) + extra, st, a);
+        return;
+    }
+    const int64_t B = kBatch / n;
+    const dim3 grid = kRows ? dim3((unsigned)tt::ceil_div(rows, B))
+                            : dim3((unsigned)tt::ceil_div(plan->nxh, B), (unsigned)(MODE == kPassY ? plan->nz : plan->ny));
+    const size_t sm = smem_fixed(n) + extra;
     switch (n) {
         case 128: hipLaunchKernelGGL((fft_pass_kernel<MODE, 128>), grid, dim3(kThreads), sm, st, a); break;
         case 192: hipLaunchKernelGGL((fft_pass_kernel<MODE, 192>), grid, dim3(kThreads), sm, st, a); break;
         case 256: hipLaunchKernelGGL((fft_pass_kernel<MODE, 256>), grid, dim3(kThreads), sm, st, a); break;
         case 384: hipLaunchKernelGGL((fft_pass_kernel<MODE, 384>), grid, dim3(kThreads), sm, st, a); break;
         case 512: hipLaunchKernelGGL((fft_pass_kernel<MODE, 512>), grid, dim3(kThreads), sm, st, a); break;
-        case 1024: hipLaunchKernelGGL((fft_pass_kernel<MODE, 1024>), grid, dim3(kThreads), sm, st, a); break;
-        default: hipLaunchKernelGGL((fft_pass_kernel<MODE, 0>), grid, dim3(kThreads), sm, st, a); break;
+        default: hipLaunchKernelGGL((fft_pass_kernel<MODE, 1024>), grid, dim3(kThreads), sm, st, a); break;
     }
 }
 
@@ -826,37 +923,15 @@ int run_passes(tt_fft_plan plan, PassArgs a, bool native, void *workspace, float
     a.out = out;
     a.sumsq = sumsq;
     a.scale = (float)(1.0 / ((double)plan->nx * plan->ny * plan->nz));
-    // pass Z (with generation)
-    a.ap = plan->ax[2];
-    a.tw = plan->tw[2];
-    a.B = pencils_per_block(plan->nz);
-    {
-        dim3 grid((unsigned)tt::ceil_div(plan->nxh, a.B), (unsigned)plan->ny);
-        const size_t sm = smem_bytes(plan->nz, a.B);
-        if (native)
-            launch_pass<kGenNative>(plan->nz, grid, sm, st, a);
-        else
-            launch_pass<kGenNoise>(plan->nz, grid, sm, st, a);
-        TT_LAUNCH_CHECK("field pass Z launch");
-    }
-    // pass Y
-    a.ap = plan->ax[1];
-    a.tw = plan->tw[1];
-    a.B = pencils_per_block(plan->ny);
-    {
-        dim3 grid((unsigned)tt::ceil_div(plan->nxh, a.B), (unsigned)plan->nz);
-        launch_pass<kPassY>(plan->ny, grid, smem_bytes(plan->ny, a.B), st, a);
-        TT_LAUNCH_CHECK("field pass Y launch");
-    }
-    // pass X
-    a.ap = plan->ax[0];
-    a.tw = plan->tw[0];
-    a.B = pencils_per_block(plan->nx);
-    {
-        dim3 grid((unsigned)tt::ceil_div((int64_t)plan->ny * plan->nz, a.B));
-        launch_pass<kPassX>(plan->nx, grid, smem_bytes(plan->nx, a.B), st, a);
-        TT_LAUNCH_CHECK("field pass X launch");
-    }
+    if (native)
+        launch_pass<kGenNative>(plan, 2, st, a);
+    else
+        launch_pass<kGenNoise>(plan, 2, st, a);
+    TT_LAUNCH_CHECK("field pass Z launch");
+    launch_pass<kPassY>(plan, 1, st, a);
+    TT_LAUNCH_CHECK("field pass Y launch");
+    launch_pass<kPassX>(plan, 0, st, a);
+    TT_LAUNCH_CHECK("field pass X launch");
     return TT_OK;
 }
 
@@ -915,26 +990,12 @@ extern "C" int tt_power_spectrum(tt_fft_plan plan, const float *field, int32_t m
     a.pscale = 1.0 / (nt * nt);
     a.hsum = sums;
     a.hcnt = counts;
-    // pass X: real rows -> half spectrum
-    a.ap = plan->ax[0];
-    a.tw = plan->tw[0];
-    a.B = pencils_per_block(plan->nx);
-    launch_pass<kFwdX>(plan->nx, dim3((unsigned)tt::ceil_div((int64_t)plan->ny * plan->nz, a.B)),
-                       smem_bytes(plan->nx, a.B), st, a);
+    launch_pass<kFwdX>(plan, 0, st, a);  // real rows -> half spectrum
     TT_LAUNCH_CHECK("power spectrum pass X launch");
-    // pass Y
-    a.ap = plan->ax[1];
-    a.tw = plan->tw[1];
-    a.B = pencils_per_block(plan->ny);
-    launch_pass<kPassY>(plan->ny, dim3((unsigned)tt::ceil_div(plan->nxh, a.B), (unsigned)plan->nz),
-                        smem_bytes(plan->ny, a.B), st, a);
+    launch_pass<kPassY>(plan, 1, st, a);
     TT_LAUNCH_CHECK("power spectrum pass Y launch");
     // pass Z with |F|^2 binning (sums and counts are ADDED to)
-    a.ap = plan->ax[2];
-    a.tw = plan->tw[2];
-    a.B = pencils_per_block(plan->nz);
-    const size_t sm = smem_bytes(plan->nz, a.B) + 2 * (size_t)nbins * sizeof(double);
-    launch_pass<kPowZ>(plan->nz, dim3((unsigned)tt::ceil_div(plan->nxh, a.B), (unsigned)plan->ny), sm, st, a);
+    launch_pass<kPowZ>(plan, 2, st, a, 2 * (size_t)nbins * sizeof(double));
     TT_LAUNCH_CHECK("power spectrum pass Z launch");
     return TT_OK;
 }
