@@ -1049,7 +1049,7 @@ __device__ __forceinline__ void time_rhs(const TraceArgs &a, const double (&y)[7
 
 // Dormand-Prince 5(4) tableau: stage nodes are implied by the rows; the last
 // row is the fifth-order solution (and its stage the next step's first, FSAL)
-__constant__ double kDPA[6][6] = {
+constexpr double kDPA[6][6] = {
     {1.0 / 5, 0, 0, 0, 0, 0},
     {3.0 / 40, 9.0 / 40, 0, 0, 0, 0},
     {44.0 / 45, -56.0 / 15, 32.0 / 9, 0, 0, 0},
@@ -1057,9 +1057,9 @@ __constant__ double kDPA[6][6] = {
     {9017.0 / 3168, -355.0 / 33, 46732.0 / 5247, 49.0 / 176, -5103.0 / 18656, 0},
     {35.0 / 384, 0, 500.0 / 1113, 125.0 / 192, -2187.0 / 6784, 11.0 / 84}};
 // fifth-order minus fourth-order weights, over the seven stages
-__constant__ double kDPE[7] = {71.0 / 57600, 0, -71.0 / 16695, 71.0 / 1920, -17253.0 / 339200, 22.0 / 525, -1.0 / 40};
+constexpr double kDPE[7] = {71.0 / 57600, 0, -71.0 / 16695, 71.0 / 1920, -17253.0 / 339200, 22.0 / 525, -1.0 / 40};
 
-// ray t of a (the order's t-th) if its status is `only` (or a has none)
+// ray t of a (the order's t-th) if its status is `only` (or a has none), by one lane
 __device__ void trace_time_ray(const TraceArgs &a, int64_t t, int32_t only) {
     const int64_t r = a.order ? (int64_t)a.order[t] : t;
     if (a.status && a.status[r] != only) return;
@@ -1142,9 +1142,214 @@ __device__ void trace_time_ray(const TraceArgs &a, int64_t t, int32_t only) {
     if (a.status) a.status[r] = bad ? 2 : 3;
 }
 
+// Few rays: four lanes a ray.  A ray is a chain of some thousand tries, so a
+// set that leaves SIMDs idle takes as long as one ray, and that is the
+// instructions of a try (one wave a SIMD issues one in about five cycles).  Lane
+// q of a quad holds axis q of position and velocity and channel q of the field,
+// lane 3 the phase, and the quad shares what a thread of its own does seven
+// times.  Every sum keeps the order of the one-lane form, and every quotient its
+// form, so both give the same bits (the accept / reject decisions would turn a
+// last-bit difference into one of the order of the tolerance).
+// Measured on a 101^3 liner that turns every ray back (1190 tries a ray): 16000
+// rays 7.25 -> 2.91 ms, 20000 (some SIMDs with two waves) 7.26 -> 4.63, 30000
+// 7.3 -> 4.8, 40000 7.35 -> 7.0, 100000 13.4 -> 15.3.  So up to kTimeQuadRays,
+// two waves on each of the 1024 SIMDs; one lane a ray beyond.
+constexpr int64_t kTimeQuadRays = 32768;
+
+// v of lanes A, B, C, D of each quad, in its lanes 0 to 3
+template <int A, int B, int C, int D>
+__device__ __forceinline__ int quad(int v) {
+    return __builtin_amdgcn_mov_dpp(v, A | B << 2 | C << 4 | D << 6, 0xf, 0xf, true);
+}
+template <int A, int B, int C, int D>
+__device__ __forceinline__ double quad(double v) {
+    return __hiloint2double(quad<A, B, C, D>(__double2hiint(v)), quad<A, B, C, D>(__double2loint(v)));
+}
+__device__ __forceinline__ bool quad_any(bool v) {
+    int f = v;
+    f |= quad<1, 0, 3, 2>(f);
+    f |= quad<2, 3, 0, 1>(f);
+    return f != 0;
+}
+
+// One lane's part of a ray: axis q of its position and velocity (q < 3), or
+// its phase as U (q = 3), and channel q of the field
+struct TimeLane {
+    bool phase;               // q = 3
+    double org, size, inv;    // the axis' first node, spacing and its reciprocal
+    double top;               // n - 1
+    double last;              // n - 2
+    const __attribute__((address_space(1))) float *field;
+};
+
+// Channel q of the field at the nodes of a position's cell, where it is in the
+// cell along axis q, and whether it is outside the grid
+struct TimeCell {
+    float v[8];
+    double t;
+    bool out;
+};
+
+// the cell of the position whose component q is X
+__device__ __forceinline__ TimeCell time_cell(const TraceArgs &a, const TimeLane &L, double X) {
+    TimeCell C;
+    const double d = X - L.org;
+    const double p0 = d * L.inv;
+    const double p = fma(fma(-p0, L.size, d), L.inv, p0);  // d / size, as the division instructions form it
+    C.out = quad_any(!L.phase && !(p >= 0.0 && p <= L.top));
+    const int i = (int)fmin(fmax(p, 0.0), L.last);  // 0 for a NaN
+    C.t = p - i;
+    const int64_t node = 4 * node_index(a, quad<0, 0, 0, 0>(i), quad<1, 1, 1, 1>(i), quad<2, 2, 2, 2>(i));
+    const auto *f = L.field + node;
+    const int64_t row = 4 * (int64_t)a.nx, plane = 4 * (int64_t)a.plane;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) C.v[c] = f[((c & 1) ? 4 : 0) + ((c & 2) ? row : 0) + ((c & 4) ? plane : 0)];
+    return C;
+}
+
+// channel q of g / dz there
+__device__ __forceinline__ double time_field(const TimeCell &C, double idz) {
+    const double tx = quad<0, 0, 0, 0>(C.t), ty = quad<1, 1, 1, 1>(C.t), tz = quad<2, 2, 2, 2>(C.t);
+    double g = 0.0;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const double w = ((c & 1) ? tx : 1.0 - tx) * ((c & 2) ? ty : 1.0 - ty) * ((c & 4) ? tz : 1.0 - tz);
+        g = fma(w, (double)C.v[c], g);
+    }
+    return (C.out ? 0.0 : g) * idz;
+}
+
+// U . U of the ray in all its lanes, added from axis A to B to z
+template <int A, int B>
+__device__ __forceinline__ double time_speed2(double U) {
+    const double m = __dmul_rn(U, U);
+    const double n = fma(U, U, quad<A, A, A, A>(m));
+    return quad<2, 2, 2, 2>(fma(U, U, quad<B, B, B, B>(n)));
+}
+
+// sum of c_j k_j, j < n
+__device__ __forceinline__ double time_dot(const double *c, const double *k, int n) {
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < n; ++j)
+        if (c[j] != 0.0) s = fma(c[j], k[j], s);
+    return s;
+}
+
+// ray r of a
+__device__ __forceinline__ void trace_time_quad(const TraceArgs &a, int64_t r) {
+    const int q = threadIdx.x & 3, ax = min(q, 2);
+    TimeLane L;
+    L.phase = q == 3;
+    L.org = ax == 0 ? a.x0 : ax == 1 ? a.y0 : a.z0;
+    L.size = ax == 0 ? a.dx : ax == 1 ? a.dy : a.dz;
+    L.inv = __builtin_amdgcn_rcp(L.size);
+    for (int i = 0; i < 2; ++i) L.inv = fma(L.inv, fma(-L.size, L.inv, 1.0), L.inv);
+    L.top = ax == 0 ? (double)a.fx1 : ax == 1 ? (double)a.fy1 : (double)a.fz1;
+    L.last = (ax == 0 ? a.nx : ax == 1 ? a.ny : a.nz) - 2;
+    L.field = (const __attribute__((address_space(1))) float *)(const void *)a.field + q;
+    const double *s = a.s0 + r;
+    double X = s[ax * a.ld_s0], U = s[(3 + ax) * a.ld_s0] / tt::kC;
+    const double nanv = __longlong_as_double(0x7ff8000000000000ll);
+    bool bad = quad_any(isnan(X) || isnan(U));
+    if (L.phase) U = 0.0;
+    if (!bad) {
+        const double hmax = 0.5 * fmin(a.dx, fmin(a.dy, a.dz));
+        const double idz = 1.0 / a.dz;
+        const double lo = L.org, hi = L.org + L.top * L.size;
+        double kx[7], ku[7];
+        kx[0] = U;
+        const double s0 = sqrt(time_speed2<1, 0>(U));
+        ku[0] = time_field(time_cell(a, L, X), idz) * (L.phase ? s0 : 1.0);
+        double tau = 0.0, h = hmax;
+        int tries = 0;
+        while (tau < a.cT) {
+            // outside the grid and moving away from it
+            if (quad_any(!L.phase && ((X < lo && U <= 0.0) || (X > hi && U >= 0.0)))) break;
+            if (++tries > kTimeMaxSteps) {
+                bad = true;
+                break;
+            }
+            const double hh = fmin(h, a.cT - tau);
+            // The phase lane's slope is its channel times |U|.  No stage
+            // depends on it, so the stages leave the factor out (that lane's
+            // kx, and X, hold no meaning) and it goes in after the last: the
+            // roots of four stages at once, one in each lane.
+            // A stage's position takes the slopes of two stages before, so its
+            // cell is loaded before the last stage's is used.
+            double Xn = fma(hh, time_dot(kDPA[0], kx, 1), X), Un, v2[7];
+            TimeCell C = time_cell(a, L, Xn);
+#pragma unroll
+            for (int st = 1; st <= 6; ++st) {
+                Un = fma(hh, time_dot(kDPA[st - 1], ku, st), U);
+                kx[st] = Un;
+                TimeCell N;
+                if (st < 6) {
+                    Xn = fma(hh, time_dot(kDPA[st], kx, st + 1), X);
+                    N = time_cell(a, L, Xn);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                ku[st] = time_field(C, idz);
+                v2[st] = st == 1 ? time_speed2<1, 0>(Un) : time_speed2<0, 1>(Un);
+                C = N;
+            }
+            const double s14 = sqrt(q == 0 ? v2[1] : q == 1 ? v2[2] : q == 2 ? v2[3] : v2[4]);
+            const double s56 = sqrt(q == 0 ? v2[5] : v2[6]);
+            const double sp[6] = {quad<0, 0, 0, 0>(s14), quad<1, 1, 1, 1>(s14), quad<2, 2, 2, 2>(s14), s14,
+                                  quad<0, 0, 0, 0>(s56), s56};
+#pragma unroll
+            for (int st = 1; st <= 6; ++st) ku[st] *= L.phase ? sp[st - 1] : 1.0;
+            Un = fma(hh, time_dot(kDPA[5], ku, 6), U);
+            // the largest scaled error estimate, over the quad
+            const double ex = L.phase ? 0.0 : time_dot(kDPE, kx, 7), eu = time_dot(kDPE, ku, 7);
+            const double su = L.phase ? kTimeTol * fmax(1.0, fmax(fabs(U), fabs(Un))) : kTimeTol;
+            double en = fmax(fabs(hh * ex) / (kTimeTol * L.size), fabs(hh * eu) / su);
+            en = fmax(en, quad<1, 0, 3, 2>(en));
+            en = fmax(en, quad<2, 3, 0, 1>(en));
+            double fac = 0.9 * pow(fmax(en, 1e-10), -0.2);
+            fac = fmin(5.0, fmax(0.2, fac));
+            if (en <= 1.0) {  // accept: the last stage is the next step's first
+                X = Xn;
+                U = Un;
+                kx[0] = kx[6];
+                ku[0] = ku[6];
+                tau += hh;
+            } else {
+                fac = fmin(fac, 1.0);
+            }
+            h = fmin(hh * fac, hmax);
+        }
+        if (!bad && tau < a.cT && !L.phase) X = fma(a.cT - tau, U, X);  // straight to cT (no field acts any more)
+    }
+    // ray_at_exit (PT:333-380): back-project to the exit plane z = z.max()
+    const double ze = a.z0 + (double)a.fz1 * a.dz;
+    const double W = quad<2, 2, 2, 2>(U);
+    const double tbp = (quad<2, 2, 2, 2>(X) - ze) / W;
+    if (q < 2) {
+        double *rf = a.rf + r + 2 * q * a.ld_rf;
+        rf[0] = bad ? nanv : X - U * tbp;
+        rf[a.ld_rf] = bad ? nanv : atan(U / W);
+    }
+    if (a.phase && L.phase) a.phase[r] = bad ? nanv : U;
+    if (a.sf && !L.phase) {
+        a.sf[r + q * a.ld_sf] = bad ? nanv : X;
+        a.sf[r + (3 + q) * a.ld_sf] = bad ? nanv : tt::kC * U;
+    }
+    if (a.status && L.phase) a.status[r] = bad ? 2 : 3;
+}
+
+// a lane per ray
 __global__ __launch_bounds__(256) void trace_time_kernel(TraceArgs a, int32_t only) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < a.n) trace_time_ray(a, t, only);
+}
+
+// four lanes per ray
+__global__ __launch_bounds__(256) void trace_time_quad_kernel(TraceArgs a, int32_t only) {
+    const int64_t t = (int64_t)blockIdx.x * (blockDim.x / 4) + threadIdx.x / 4;
+    if (t >= a.n) return;
+    const int64_t r = a.order ? (int64_t)a.order[t] : t;
+    if (!a.status || a.status[r] == only) trace_time_quad(a, r);
 }
 
 // the rays of a batch the z-march handed over (status 1): one block per chunk
@@ -1306,8 +1511,12 @@ extern "C" int tt_trace_time(const float *field4, const tt_grid *grid, const tt_
     a.sf = sf;
     a.ld_sf = ld_sf;
     a.status = status;
-    hipLaunchKernelGGL(trace_time_kernel, dim3((unsigned)tt::ceil_div(n, 256)), dim3(256), 0, tt::as_stream(stream), a,
-                       only_status);
+    if (n <= kTimeQuadRays)
+        hipLaunchKernelGGL(trace_time_quad_kernel, dim3((unsigned)tt::ceil_div(n, 64)), dim3(256), 0,
+                           tt::as_stream(stream), a, only_status);
+    else
+        hipLaunchKernelGGL(trace_time_kernel, dim3((unsigned)tt::ceil_div(n, 256)), dim3(256), 0,
+                           tt::as_stream(stream), a, only_status);
     TT_LAUNCH_CHECK("tt_trace_time launch");
     return TT_OK;
 }
