@@ -193,7 +193,7 @@ int tt_trace_rk4_counted(const float *field4, const tt_grid *grid, const tt_trac
                          int64_t ld_rf, double *phase, int32_t *status, void *stream);
 
 /* Ensembles: the rays of many realisations (uneven grids and ray counts)
- * traced in ONE persistent launch.  No reference counterpart as a call: it
+ * traced in ONE launch.  No reference counterpart as a call: it
  * replaces running ElectronCube.solve once per realisation, as the reference's
  * drivers do in a loop or across MPI ranks (particle_tracking/
  * example_multiprocess.py:41-62, example_MPI.py:82-149).  Each item is one
@@ -205,9 +205,9 @@ int tt_trace_rk4_counted(const float *field4, const tt_grid *grid, const tt_trac
  * items and a chunk table (chunk rays per entry, items with the most z-steps
  * first) into `workspace` with synchronous copies and fills `info`;
  * tt_batch_trace is stream-ordered and allocation-free, so it can be captured
- * in a graph: it resets the chunk counter with a kernel and launches
- * blocks_per_cu (0 = the occupancy limit) x CUs blocks that take chunks until
- * none is left.  Results equal tt_trace_rk4's for the same variant. */
+ * in a graph: it launches a block for every `block` rays of each chunk, in the
+ * table's order, at most blocks_per_cu (0 = the occupancy limit) of them on a CU
+ * at a time.  Results equal tt_trace_rk4's for the same variant. */
 typedef struct {
     const float *field4;
     tt_grid grid;
@@ -228,7 +228,7 @@ typedef struct {
 
 typedef struct {
     int32_t block;         /* threads per block: 64, 128 or 256 */
-    int32_t blocks_per_cu; /* persistent blocks per CU, 0 = occupancy limit */
+    int32_t blocks_per_cu; /* at most so many blocks on a CU at a time, 0 = occupancy limit */
     int32_t variant;       /* 0 cell-cached, 1 per-stage gathers (as tt_trace_opts) */
 } tt_batch_tuning;
 

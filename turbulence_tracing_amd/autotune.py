@@ -3,7 +3,7 @@ settings on the device, and remembers the winner per device and problem.
 
 The reference has no counterpart (it runs one configuration of numpy and
 scipy).  The tuned quantities here are the tracer's launch shape (threads per
-block, persistent blocks per CU, rays per work chunk), its kernel variant
+block, resident blocks per CU, rays per work chunk), its kernel variant
 (cell-cached or per-stage gathers) and the ray-ordering brick (entry columns
 grouped in bricks of 2^shift cells), which sets how coherent the field gathers
 of a wavefront are.  Candidates are timed with HIP events on the current

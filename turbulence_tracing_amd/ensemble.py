@@ -1,5 +1,5 @@
 """Batched ensembles: many turbulence realisations of uneven size traced in
-one persistent launch, the whole ensemble step captured in one HIP graph.
+one launch, the whole ensemble step captured in one HIP graph.
 
 The reference runs realisations one after another (its drivers loop over
 seeds or spread them over processes, particle_tracking/
@@ -7,9 +7,8 @@ example_multiprocess.py:41-62, example_MPI.py:82-149), each through
 gaussian3D_FFT, calc_dndr, init_beam, solve and the detectors.  Here every
 member keeps its own resident buffers (a Pipeline), the per-member stages
 (field, gradient, beam, ray order, detectors) are stream-ordered launches, and
-the rays of all members go through one persistent tracer launch
-(tt_batch_trace) whose blocks take work chunks from a device counter, longest
-rays first.  The launch shape, kernel variant and ray-ordering brick come from
+the rays of all members go through one tracer launch (tt_batch_trace) whose
+blocks cover the members' chunks of rays, longest rays first.  The launch shape, kernel variant and ray-ordering brick come from
 the project's autotuner.  After one eager step the whole step is captured in
 a torch CUDA graph (a hipGraph on ROCm) and replayed.
 """
