@@ -96,6 +96,18 @@ __device__ __forceinline__ void dft<3>(float2 *v) {
     v[2] = csub(m, su);
 }
 
+// the same with the last output's product rounded before its difference
+__device__ __forceinline__ void dft3_pow(float2 *v) {
+#pragma clang fp contract(off)
+    const float c = -0.5f, s = 0.86602540378443865f;
+    const float2 a = v[0], b = v[1], d = v[2];
+    const float2 t = cadd(b, d), u = csub(b, d);
+    const float2 m = make_float2(fmaf(c, t.x, a.x), fmaf(c, t.y, a.y));
+    v[0] = cadd(a, t);
+    v[1] = make_float2(fmaf(-s, u.y, m.x), fmaf(s, u.x, m.y));
+    v[2] = make_float2(m.x - -s * u.y, m.y - s * u.x);
+}
+
 template <>
 __device__ __forceinline__ void dft<5>(float2 *v) {
     const float c1 = 0.30901699437494742f, s1 = 0.95105651629515357f;   // 2 pi / 5
@@ -222,7 +234,7 @@ __device__ __forceinline__ void first_pass(float2 *buf, Load load) {
 }
 
 // last pass (Ns = N / R): outputs are elements b + NS q of pencil p
-template <int N, int NS, bool PFAST, class Store>
+template <int N, int NS, bool PFAST, bool POW, class Store>
 __device__ __forceinline__ void last_pass(const float2 *buf, const float2 *tw, Store store) {
     constexpr int R = N / NS, B = kBatch / N, TOT = B * NS;
     constexpr int PER = (TOT + kThreads - 1) / kThreads;
@@ -239,29 +251,62 @@ __device__ __forceinline__ void last_pass(const float2 *buf, const float2 *tw, S
 #pragma unroll
                 for (int r = 1; r < R; ++r) v[r] = cmul(v[r], tw[r * b]);
             }
-            dft<R>(v);
+            if constexpr (POW && R == 3)
+                dft3_pow(v);
+            else
+                dft<R>(v);
 #pragma unroll
             for (int q = 0; q < R; ++q) store(p, b + NS * q, v[q]);
         }
     }
 }
 
-template <int N, int NS, bool PFAST, class Store>
+template <int N, int NS, bool PFAST, bool POW, class Store>
 __device__ __forceinline__ void rest_passes(float2 *buf, const float2 *tw, Store store) {
     constexpr int R = radix_at<N, NS>();
     if constexpr (NS * R == N) {
-        last_pass<N, NS, PFAST>(buf, tw, store);
+        last_pass<N, NS, PFAST, POW>(buf, tw, store);
     } else {
         pass_r_body<R>(buf, N, N + 1, kBatch / N, NS, tw);
-        rest_passes<N, NS * R, PFAST>(buf, tw, store);
+        rest_passes<N, NS * R, PFAST, POW>(buf, tw, store);
+    }
+}
+
+// outputs a thread has in the last pass, at most
+template <int N, int NS = 1>
+constexpr int outputs_of() {
+    constexpr int R = radix_at<N, NS>();
+    if constexpr (NS * R == N)
+        return (kBatch / N * NS + kThreads - 1) / kThreads * R;
+    else
+        return outputs_of<N, NS * R>();
+}
+// f(p, j) over them, in the order the last pass stores them
+template <int N, bool PFAST, int NS = 1, class F>
+__device__ __forceinline__ void each_output(F f) {
+    constexpr int R = radix_at<N, NS>();
+    if constexpr (NS * R == N) {
+        constexpr int B = kBatch / N, TOT = B * NS, PER = (TOT + kThreads - 1) / kThreads;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int beta = threadIdx.x + i * kThreads;
+            if (TOT % kThreads == 0 || beta < TOT) {
+                int p, b;
+                split_bf<B, NS, PFAST>(beta, p, b);
+#pragma unroll
+                for (int q = 0; q < R; ++q) f(p, b + NS * q);
+            }
+        }
+    } else {
+        each_output<N, PFAST, NS * R>(f);
     }
 }
 
 // the whole transform of the block's B pencils: load(p, j) -> store(p, j, v)
-template <int N, bool PFAST, class Load, class Store>
+template <int N, bool PFAST, bool POW = false, class Load, class Store>
 __device__ __forceinline__ void fft_pow2(float2 *buf, const float2 *tw, Load load, Store store) {
     first_pass<N, PFAST>(buf, load);
-    rest_passes<N, radix_at<N, 1>(), PFAST>(buf, tw, store);
+    rest_passes<N, radix_at<N, 1>(), PFAST, POW>(buf, tw, store);
 }
 
 enum { kGenNative = 0, kGenNoise = 1, kPassY = 2, kPassX = 3, kFwdX = 4, kPowZ = 5 };
@@ -286,8 +331,8 @@ struct PassArgs {
     const float *in;
     int mode, nbins;
     double fz_step, fy_step, fx_step;  // 1 / (n dx) per axis (spectrum_3D_scalar frequencies)
-    double bin_w;                      // bin width in |k| (spectrum_3D_scalar)
-    double pscale;                     // factor on |F|^2 (compute3Dspectrum: 1 / nt^2)
+    double bin_w, inv_bin_w;           // bin width in |k| (spectrum_3D_scalar)
+    double pscale;                     // factor on |F|^2 (compute3Dspectrum: 1 / nt^2, else 1)
     double *hsum, *hcnt;
 };
 
@@ -375,38 +420,119 @@ __device__ __forceinline__ int loop_value(int j, int n) {
     return j <= hi ? j : j - n;
 }
 
+// The bins an element's power goes to: w0 times to b0 and, where its mirror's
+// bin is another one, once to b1 (-1: none).
+struct Bins {
+    int b0, b1;
+    uint32_t w0;
+};
 #pragma clang fp contract(off)
-__device__ __forceinline__ void bin_power(const PassArgs &a, int jx, int jy, int jz, float power, double *hs,
-                                          double *hc) {
+__device__ __forceinline__ Bins bins_of(const PassArgs &a, int jx, int jy, int jz) {
     const bool self_conj = jx == 0 || (a.nx % 2 == 0 && jx == a.nx / 2);
     if (a.mode == 0) {
         const double f0 = (double)signed_of(jz, a.nz) * a.fz_step;
         const double f1 = (double)signed_of(jy, a.ny) * a.fy_step;
         const double f2 = (double)signed_of(jx, a.nx) * a.fx_step;
         const double K = sqrt((f0 * f0 + f1 * f1) + f2 * f2);
-        int b = (int)(K / a.bin_w);
+        int b = (int)(K * a.inv_bin_w);  // at most one off: corrected by the comparisons
         if (K < (double)b * a.bin_w) --b;
         else if (K >= (double)(b + 1) * a.bin_w) ++b;
-        if (b < 0 || b > a.nbins - 2) return;
-        const double w = self_conj ? 1.0 : 2.0;
-        atomicAdd(&hs[b], w * (double)power);
-        atomicAdd(&hc[b], w);
-        return;
+        return Bins{b <= a.nbins - 2 ? b : -1, -1, self_conj ? 1u : 2u};
     }
-    const double p = (double)power * a.pscale;
-    for (int m = 0; m < (self_conj ? 1 : 2); ++m) {
-        const int ix = m ? (a.nx - jx) % a.nx : jx, iy = m ? (a.ny - jy) % a.ny : jy, iz = m ? (a.nz - jz) % a.nz : jz;
+    const auto shell = [&](int ix, int iy, int iz) {
         const int v0 = loop_value(iz, a.nz), v1 = loop_value(iy, a.ny), v2 = loop_value(ix, a.nx);
-        if (v0 == INT_MIN || v1 == INT_MIN || v2 == INT_MIN) continue;
-        const double rk = sqrt((double)v0 * v0 + (double)v1 * v1 + (double)v2 * v2);
-        const int sh = (int)rint(rk);
-        if (sh < a.nbins) {
-            atomicAdd(&hs[sh], p);
-            atomicAdd(&hc[sh], 1.0);
-        }
-    }
+        if (v0 == INT_MIN || v1 == INT_MIN || v2 == INT_MIN) return -1;
+        // round(sqrt(s2)) is the integer b with b (b - 1) < s2 <= b (b + 1)
+        const int s2 = v0 * v0 + v1 * v1 + v2 * v2;
+        int b = (int)(__builtin_amdgcn_sqrtf((float)s2) + 0.5f);
+        if (s2 > b * (b + 1)) ++b;
+        if (b > 0 && s2 <= b * (b - 1)) --b;
+        return b < a.nbins ? b : -1;
+    };
+    const int b0 = shell(jx, jy, jz);
+    if (self_conj) return Bins{b0, -1, 1u};
+    const int b1 = shell(jx ? a.nx - jx : 0, jy ? a.ny - jy : 0, jz ? a.nz - jz : 0);
+    return b0 == b1 ? Bins{b0, -1, 2u} : Bins{b0, b1, 1u};
 }
 #pragma clang fp contract(on)
+
+// A block's histogram.  Lanes next to each other hold neighbouring kx, whose
+// power goes to a few bins, and LDS adds to one address wait for each other: so
+// lanes spread their adds over up to 16 copies (lane mod copies; as many as the
+// FFT's buffer, free by then, has room for), which are summed per tile into the
+// block's own.  A block takes several tiles and adds its histogram to the result
+// once: those adds go to the same few addresses from every block.  Counts are
+// integers in LDS.  Bound by the adds and the bins' arithmetic: pass Z and the two
+// before it took 169 us (mode 0) and 188 (mode 1) at 256^3 with adds straight to
+// the block's own bins, a tile a block, and a double quotient, root and integer
+// remainders an element; 134 and 140 now, 512^3 983 and 1214 -> 888 and 910.
+// 512 blocks: two a CU, which is what the tile loop's registers let run (1024:
+// 142 and 148; a tile a block 144 and 151).
+constexpr int kPowBlocks = 512;
+extern __shared__ float2 smem[];
+struct Histogram {
+    // places in LDS, in eight and in four bytes (kept as numbers: through
+    // pointers held here the adds become flat ones): the block's sums and
+    // counts, the copies' (`stride` apart)
+    int hs, hc, cs, cc;
+    int nbins, copies, stride;
+    double scale;
+    static __device__ __forceinline__ double &f64(int at) { return reinterpret_cast<double *>(smem)[at]; }
+    static __device__ __forceinline__ uint32_t &u32(int at) { return reinterpret_cast<uint32_t *>(smem)[at]; }
+    // own: where the block's histogram begins; spare, bytes: room for copies
+    __device__ Histogram(const PassArgs &a, int own, int spare, int bytes)
+        : hs(own), hc(2 * (own + a.nbins)), nbins(a.nbins), copies(16), stride(a.nbins | 1), scale(a.pscale) {
+        while (copies > 1 && copies * stride * 12 > bytes) copies /= 2;
+        cs = copies > 1 ? spare : hs;
+        cc = copies > 1 ? 2 * (spare + copies * stride) : hc;
+    }
+    __device__ void clear_own(int threads) const {
+        for (int j = threadIdx.x; j < nbins; j += threads) {
+            f64(hs + j) = 0.0;
+            u32(hc + j) = 0u;
+        }
+    }
+    __device__ void clear_copies(int threads) const {
+        if (copies > 1)
+            for (int j = threadIdx.x; j < copies * stride; j += threads) {
+                f64(cs + j) = 0.0;
+                u32(cc + j) = 0u;
+            }
+    }
+    // power: |F|^2
+    __device__ __forceinline__ void add(const Bins &b, float power) const {
+        const double p = (double)power * scale;
+        const int at = (int)(threadIdx.x & (copies - 1)) * stride;
+        if (b.b0 >= 0) {
+            atomicAdd(&f64(cs + at + b.b0), b.w0 == 2 ? p + p : p);
+            atomicAdd(&u32(cc + at + b.b0), b.w0);
+        }
+        if (b.b1 >= 0) {
+            atomicAdd(&f64(cs + at + b.b1), p);
+            atomicAdd(&u32(cc + at + b.b1), 1u);
+        }
+    }
+    __device__ void sum_copies(int threads) const {
+        if (copies > 1)
+            for (int j = threadIdx.x; j < nbins; j += threads) {
+                double t = 0.0;
+                uint32_t c = 0;
+                for (int k = 0; k < copies; ++k) {
+                    t += f64(cs + k * stride + j);
+                    c += u32(cc + k * stride + j);
+                }
+                f64(hs + j) += t;
+                u32(hc + j) += c;
+            }
+    }
+    __device__ void flush(const PassArgs &a, int threads) const {
+        for (int j = threadIdx.x; j < nbins; j += threads)
+            if (const uint32_t c = u32(hc + j)) {
+                atomicAdd(&a.hsum[j], f64(hs + j));
+                atomicAdd(&a.hcnt[j], (double)c);
+            }
+    }
+};
 
 // add the block's sum of v to *out
 template <int THREADS>
@@ -425,32 +551,44 @@ __device__ __forceinline__ void block_sum(double v, double *out) {
 // The fixed lengths: NF points a pencil, kBatch / NF pencils a block.
 template <int MODE, int NF>
 __global__ __launch_bounds__(kThreads) void fft_pass_kernel(PassArgs a) {
-    extern __shared__ float2 smem[];
     constexpr int BF = kBatch / NF;
     float2 *buf = smem;
     float2 *tw = smem + BF * (NF + 1);
     for (int j = threadIdx.x; j < NF; j += kThreads) tw[j] = a.tw[j];
     if constexpr (MODE == kPowZ) {
-        double *hs = reinterpret_cast<double *>(tw + NF), *hc = hs + a.nbins;
-        for (int j = threadIdx.x; j < 2 * a.nbins; j += kThreads) hs[j] = 0.0;
-        const int kx0 = blockIdx.x * BF, fixed = blockIdx.y;
-        fft_pow2<NF, true>(
-            buf, tw,
-            [&](int p, int j) {
-                const int kx = kx0 + p;
-                return kx < a.nxh ? a.spec[((int64_t)j * a.ny + fixed) * a.nxh + kx] : make_float2(0.f, 0.f);
-            },
-            [&](int p, int j, float2 v) {
-                const int kx = kx0 + p;
-                if (kx < a.nxh) bin_power(a, kx, fixed, j, v.x * v.x + v.y * v.y, hs, hc);
-            });
-        __syncthreads();
-        for (int j = threadIdx.x; j < a.nbins; j += kThreads) {
-            if (hc[j] != 0.0) {
-                atomicAdd(&a.hsum[j], hs[j]);
-                atomicAdd(&a.hcnt[j], hc[j]);
+        // columns are numbered through the whole spectrum (column q begins at
+        // element q of the first plane): only the last tile is ragged
+        const int64_t plane = (int64_t)a.nxh * a.ny;
+        // The powers of a tile's elements go back to LDS (half of the FFT's
+        // buffer, the histogram's copies in the rest): taken from registers, the
+        // bins of all of a thread's elements are formed at once in 270 of them.
+        float *pw = reinterpret_cast<float *>(buf);
+        constexpr int kPw = BF * NF;
+        const Histogram H(a, BF * (NF + 1) + NF, kPw / 2, BF * (NF + 1) * 8 - kPw * 4);
+        H.clear_own(kThreads);
+        for (int64_t first = (int64_t)blockIdx.x * BF; first < plane; first += (int64_t)gridDim.x * BF) {
+            float power[outputs_of<NF>()];
+            int n = 0;
+            fft_pow2<NF, true, true>(
+                buf, tw,
+                [&](int p, int j) { return first + p < plane ? a.spec[j * plane + first + p] : make_float2(0.f, 0.f); },
+                [&](int, int, float2 v) { power[n++] = fmaf(v.x, v.x, v.y * v.y); });
+            __syncthreads();
+            n = 0;
+            each_output<NF, true>([&](int p, int j) { pw[j * BF + p] = power[n++]; });
+            H.clear_copies(kThreads);
+            __syncthreads();
+#pragma unroll 1
+            for (int e = threadIdx.x; e < kPw; e += kThreads) {
+                const int j = e / BF;
+                const uint32_t q = (uint32_t)first + (e - j * BF), ky = q / (uint32_t)a.nxh;
+                if (q < (uint32_t)plane) H.add(bins_of(a, (int)(q - ky * a.nxh), (int)ky, j), pw[e]);
             }
+            __syncthreads();
+            H.sum_copies(kThreads);
+            __syncthreads();
         }
+        H.flush(a, kThreads);
     } else if constexpr (MODE == kFwdX) {
         const int64_t rows = (int64_t)a.ny * a.nz, r0 = (int64_t)blockIdx.x * BF;
         fft_pow2<NF, false>(
@@ -634,13 +772,9 @@ __device__ __forceinline__ int outputs_per_thread(int R, int nbf, int lb) {
 
 template <int MODE>
 __global__ __launch_bounds__(kAnyThreads) __attribute__((amdgpu_waves_per_eu(6, 6))) void fft_any_kernel(PassArgs a) {
-    extern __shared__ float2 smem[];
     const int n = a.ap.n, lb = a.lb, PB = 1 << lb;
     float2 *buf = smem, *alt = smem + n * PB, *tw = alt + n * PB;
-    double *hs = reinterpret_cast<double *>(tw + n), *hc = hs + a.nbins;
     for (int j = threadIdx.x; j < n; j += kAnyThreads) tw[j] = a.tw[j];
-    if (MODE == kPowZ)
-        for (int j = threadIdx.x; j < 2 * a.nbins; j += kAnyThreads) hs[j] = 0.0;
     // pencils: columns (elements `step` apart from `base`) or rows
     constexpr bool kRows = MODE == kPassX || MODE == kFwdX;
     const int64_t first = (int64_t)blockIdx.x * PB;
@@ -730,18 +864,19 @@ __global__ __launch_bounds__(kAnyThreads) __attribute__((amdgpu_waves_per_eu(6, 
         }
         if (MODE == kPassX && a.sumsq) block_sum<kAnyThreads>(ss, a.sumsq);
     } else if constexpr (MODE == kPowZ) {
+        const Histogram H(a, (2 * PB + 1) * n, (int)(alt - smem), n * PB * 8);
+        H.clear_own(kAnyThreads);
+        H.clear_copies(kAnyThreads);
+        __syncthreads();
         if (live)
             for (int j = j0; j < n; j += dj) {
                 const float2 v = buf[at(j, p0, lb)];
-                bin_power(a, kx, ky, j, v.x * v.x + v.y * v.y, hs, hc);
+                H.add(bins_of(a, kx, ky, j), fmaf(v.x, v.x, v.y * v.y));
             }
         __syncthreads();
-        for (int j = threadIdx.x; j < a.nbins; j += kAnyThreads) {
-            if (hc[j] != 0.0) {
-                atomicAdd(&a.hsum[j], hs[j]);
-                atomicAdd(&a.hcnt[j], hc[j]);
-            }
-        }
+        H.sum_copies(kAnyThreads);
+        __syncthreads();
+        H.flush(a, kAnyThreads);
     } else if (live) {
         for (int j = j0; j < n; j += dj) a.spec[base + j * step] = buf[at(j, p0, lb)];
     }
@@ -889,18 +1024,19 @@ void launch_pass(tt_fft_plan plan, int ax, hipStream_t st, PassArgs a, size_t ex
     a.ap = plan->ax[ax];
     a.tw = plan->tw[ax];
     constexpr bool kRows = MODE == kPassX || MODE == kFwdX;
-    const int64_t rows = (int64_t)plan->ny * plan->nz;
+    const int64_t count = kRows ? (int64_t)plan->ny * plan->nz : (int64_t)plan->nxh * (MODE == kPassY ? plan->nz : plan->ny);
     if (!fixed_length(n)) {
         a.lb = pencils_any(n, extra);
-        const int64_t count = kRows ? rows : (int64_t)plan->nxh * (MODE == kPassY ? plan->nz : plan->ny);
         hipLaunchKernelGGL(fft_any_kernel<MODE>, dim3((unsigned)tt::ceil_div(count, (int64_t)1 << a.lb)),
                            dim3(kAnyThreads),
                            smem_any(n, a.lb) + extra, st, a);
         return;
     }
     const int64_t B = kBatch / n;
-    const dim3 grid = kRows ? dim3((unsigned)tt::ceil_div(rows, B))
-                            : dim3((unsigned)tt::ceil_div(plan->nxh, B), (unsigned)(MODE == kPassY ? plan->nz : plan->ny));
+    const dim3 grid = kRows ? dim3((unsigned)tt::ceil_div(count, B))
+                    : MODE == kPowZ
+                        ? dim3((unsigned)std::min<int64_t>(tt::ceil_div(count, B), kPowBlocks))
+                        : dim3((unsigned)tt::ceil_div(plan->nxh, B), (unsigned)(MODE == kPassY ? plan->nz : plan->ny));
     const size_t sm = smem_fixed(n) + extra;
     switch (n) {
         case 128: hipLaunchKernelGGL((fft_pass_kernel<MODE, 128>), grid, dim3(kThreads), sm, st, a); break;
@@ -986,8 +1122,9 @@ extern "C" int tt_power_spectrum(tt_fft_plan plan, const float *field, int32_t m
     a.fy_step = 1.0 / ((double)plan->ny * dx);
     a.fz_step = 1.0 / ((double)plan->nz * dx);
     a.bin_w = bin_w;
+    a.inv_bin_w = mode == 0 ? 1.0 / bin_w : 0.0;
     const double nt = (double)plan->nx * plan->ny * plan->nz;
-    a.pscale = 1.0 / (nt * nt);
+    a.pscale = mode == 0 ? 1.0 : 1.0 / (nt * nt);
     a.hsum = sums;
     a.hcnt = counts;
     launch_pass<kFwdX>(plan, 0, st, a);  // real rows -> half spectrum
