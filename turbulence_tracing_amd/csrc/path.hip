@@ -300,9 +300,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NODE ? 5 : 
     S.ph = 0.0;
     S.segx = S.segy = S.crossx = S.crossy = S.qx = S.qy = 0.f;
     S.cix = S.ciy = -1;
-    for (int q = 0; q < 2 * kSeg; ++q) f[q * a.ldf] = 0.f;
     const int iz0 = Zs >= (double)ncell ? ncell : (int)Zs;
     S.seg = (iz0 * kSeg) / (ncell > 0 ? ncell : 1);
+    // Every segment's sums are written once: zero for those before the first
+    // step and (below) behind the last, the others as the march leaves them.
+    // Zeroing all of them first cost a third of the bytes written: 1e7 rays
+    // through 512^3 in blocks of 16 1.96 -> 1.81 ms.
+    const auto no_segments = [&](int q0, int q1) {
+        for (int q = q0; q < q1; ++q) f[q * a.ldf] = f[(kSeg + q) * a.ldf] = 0.f;
+    };
+    no_segments(0, S.seg);
     S.seg_end = ((S.seg + 1) * ncell + kSeg - 1) / kSeg;
     const bool on_boundary = Zs == (double)iz0 && iz0 % a.k == 0;
     const int bstart = on_boundary ? iz0 : min(ncell, (iz0 / a.k + 1) * a.k);
@@ -370,6 +377,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NODE ? 5 : 
         f[S.seg * a.ldf] = S.segx;
         f[(kSeg + S.seg) * a.ldf] = S.segy;
     }
+    no_segments(S.seg + 1, kSeg);
     const float U = S.U, V = S.V, Wd = S.Wd, dpx = S.dpx, dpy = S.dpy;
     const double ph = S.ph;
     const double Uf = U, Vf = V, Wf = 1.0 + (double)Wd;
