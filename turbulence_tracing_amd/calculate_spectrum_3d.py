@@ -19,18 +19,24 @@ def _device_field(data, device="cuda"):
     return t.to(device=device, dtype=torch.float32).contiguous()
 
 
-def power_bins(data, dx, nbins, mode, bin_w=0.0, device="cuda"):
-    """(sums, counts) float64 device tensors of tt_power_spectrum."""
+def _power_bins(data, dx, nbins, mode, bin_w=0.0, device="cuda"):
+    """The sums and counts of tt_power_spectrum as one float64 device tensor
+    [2, nbins]: one fill and one copy to the host instead of two."""
     f = _device_field(data, device)
     m0, m1, m2 = f.shape
     plan = FieldPlan((m2, m1, m0), device)
-    sums = torch.zeros(nbins, dtype=torch.float64, device=device)
-    counts = torch.zeros(nbins, dtype=torch.float64, device=device)
+    out = torch.zeros((2, nbins), dtype=torch.float64, device=device)
     plan.lib.tt_power_spectrum(plan.handle, _lib.ptr(f), int(mode), int(nbins), float(dx), float(bin_w),
-                               _lib.ptr(plan.workspace), _lib.ptr(sums), _lib.ptr(counts), _lib.stream_ptr())
+                               _lib.ptr(plan.workspace), _lib.ptr(out[0]), _lib.ptr(out[1]), _lib.stream_ptr())
     torch.cuda.current_stream().synchronize()
     plan.close()
-    return sums, counts
+    return out
+
+
+def power_bins(data, dx, nbins, mode, bin_w=0.0, device="cuda"):
+    """(sums, counts) float64 device tensors of tt_power_spectrum."""
+    out = _power_bins(data, dx, nbins, mode, bin_w, device)
+    return out[0], out[1]
 
 
 def spectrum_3D_scalar(data, dx, k_bin_num=100):
@@ -41,8 +47,7 @@ def spectrum_3D_scalar(data, dx, k_bin_num=100):
     shape = tuple(int(s) for s in np.shape(data))
     f = [(m // 2) * (1.0 / (m * dx)) for m in shape]
     k_bin_width = np.sqrt(f[0] ** 2 + f[1] ** 2 + f[2] ** 2) / k_bin_num
-    sums, counts = power_bins(data, dx, k_bin_num, 0, k_bin_width)
-    sums, counts = sums.cpu().numpy(), counts.cpu().numpy()
+    sums, counts = _power_bins(data, dx, k_bin_num, 0, k_bin_width).cpu().numpy()
     k_bins = k_bin_width * np.arange(0, k_bin_num + 1)
     k_bins_weighted = (0.5 * (k_bins[:-1] ** 3 + k_bins[1:] ** 3)) ** (1 / 3)
     spect3D = np.zeros_like(k_bins_weighted)
