@@ -358,7 +358,6 @@ class Surrogate:
         """Adam with cosine decay on (features, normalised targets)."""
         N = feat.shape[0]
         X = self.standardize(feat)
-        fused = self._fused_step(X, target, batch, wd)
         gen = torch.Generator(device=self.device).manual_seed(seed)
         steps = epochs * (N // batch)
         loss = torch.zeros(2, dtype=torch.float64, device=self.device)
@@ -369,6 +368,8 @@ class Surrogate:
         for ep in range(epochs):
             perm = torch.randperm(N, generator=gen, device=self.device)
             loss.zero_()
+            # taken anew each epoch: `log` may load weights or replace the network between two
+            fused = self._fused_step(X, target, batch, wd)
             for b in range(N // batch):
                 idx = perm[b * batch:(b + 1) * batch]
                 lr_t = lr_min + 0.5 * (lr - lr_min) * (1 + np.cos(np.pi * st / max(1, steps)))
@@ -395,7 +396,10 @@ class Surrogate:
         launches instead of 45), or None where it does not serve: a network
         of another shape than the surrogate's, a replaced MLP class, or
         targets that are not this loss's fp32 columns on the device.  Returns
-        a function of (row indices of the batch, learning rate, loss sums)."""
+        a function of (row indices of the batch, learning rate, loss sums),
+        which holds the network's tensors and the transposes of their bf16
+        copies as they are now: nothing else may write to them while it is
+        used."""
         m = self.mlp
         if (type(m) is not MLP or len(m.dims) != 5 or m.dims[1:4] != (256, 256, 256) or m.dims[4] != NOUT or
                 m.dims[0] != NFEAT or batch < 1 or target.dtype != torch.float32 or target.device != X.device or
@@ -407,16 +411,17 @@ class Surrogate:
         self.lib.tt_mlp_train_workspace_bytes(batch, C.byref(nbytes))
         ws = torch.empty(nbytes.value, dtype=torch.uint8, device=self.device)
         a = _lib.MlpTrain()
+        layers = [(m.W[l], m.b[l], m.Wb[l], Wt[l], m.dW[l], m.db[l], m.mW[l], m.vW[l], m.mb[l], m.vb[l])
+                  for l in range(4)]
         for l in range(4):
-            a.layer[l] = _lib.MlpLayer(*(_p(t) for t in (m.W[l], m.b[l], m.Wb[l], Wt[l], m.dW[l], m.db[l], m.mW[l],
-                                                         m.vW[l], m.mb[l], m.vb[l])))
+            a.layer[l] = _lib.MlpLayer(*(_p(t) for t in layers[l]))
         a.X, a.ldx, a.T, a.ldt = _p(X), X.stride(0), _p(T), T.stride(0)
         a.batch, a.nfeat, a.n_reg, a.n_err = batch, NFEAT, N_REG, N_ERR
         a.w_reg[:N_REG] = self.w_reg.tolist()
         a.err_lo[:N_ERR], a.err_hi[:N_ERR] = self.err_lo.tolist(), self.err_hi.tolist()
         a.tau, a.b1, a.b2, a.eps, a.weight_decay = float(self.tau), 0.9, 0.999, 1e-8, float(wd)
         a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes.value
-        keep = (X, T, Wt, ws)
+        keep = (X, T, layers, ws)
 
         def step(idx, lr, loss, _keep=keep):
             m.step += 1
