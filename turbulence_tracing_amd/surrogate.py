@@ -369,7 +369,7 @@ class Surrogate:
             perm = torch.randperm(N, generator=gen, device=self.device)
             loss.zero_()
             # taken anew each epoch: `log` may load weights or replace the network between two
-            fused = self._fused_step(X, target, batch, wd)
+            fused = self._fused_step(X, target, batch, wd) if N >= batch else None
             for b in range(N // batch):
                 idx = perm[b * batch:(b + 1) * batch]
                 lr_t = lr_min + 0.5 * (lr - lr_min) * (1 + np.cos(np.pi * st / max(1, steps)))
@@ -394,16 +394,18 @@ class Surrogate:
     def _fused_step(self, X, target, batch, wd):
         """The training step as one library call (tt_mlp_train_step: three
         launches instead of 45), or None where it does not serve: a network
-        of another shape than the surrogate's, a replaced MLP class, or
-        targets that are not this loss's fp32 columns on the device.  Returns
+        of another shape than the surrogate's, a replaced MLP class, more than
+        2^24 rows a step, tensors off its 16-byte alignment, or targets that
+        are not this loss's fp32 columns on the device.  Returns
         a function of (row indices of the batch, learning rate, loss sums),
         which holds the network's tensors and the transposes of their bf16
         copies as they are now: nothing else may write to them while it is
         used."""
         m = self.mlp
         if (type(m) is not MLP or len(m.dims) != 5 or m.dims[1:4] != (256, 256, 256) or m.dims[4] != NOUT or
-                m.dims[0] != NFEAT or batch < 1 or target.dtype != torch.float32 or target.device != X.device or
-                target.dim() != 2 or target.shape[1] != N_REG or target.shape[0] < X.shape[0]):
+                m.dims[0] != NFEAT or not 1 <= batch <= 1 << 24 or any(t.data_ptr() % 16 for t in (*m.Wb, *m.b)) or
+                target.dtype != torch.float32 or target.device != X.device or target.dim() != 2 or
+                target.shape[1] != N_REG or target.shape[0] < X.shape[0]):
             return None
         T = target if target.stride(1) == 1 and target.stride(0) >= N_REG else target.contiguous()
         Wt = [None] + [w.t().contiguous() for w in m.Wb[1:]]
