@@ -202,8 +202,8 @@ int tt_trace_rk4_counted(const float *field4, const tt_grid *grid, const tt_trac
  * does after tt_trace_rk4 (light-travel budget cT, m, as in tt_trace_opts),
  * in a second launch of the same call; without one they are NaN.
  * tt_batch_prepare uploads the
- * items and a chunk table (chunk rays per entry, items with the most z-steps
- * first) into `workspace` with synchronous copies and fills `info`;
+ * items and a chunk table (chunk rays per entry, rounded up to a multiple of
+ * 256 and no more than the largest item's; items with the most z-steps first) into `workspace` with synchronous copies and fills `info`;
  * tt_batch_trace is stream-ordered and allocation-free, so it can be captured
  * in a graph: it launches a block for every `block` rays of each chunk, in the
  * table's order, at most blocks_per_cu (0 = the occupancy limit) of them on a CU

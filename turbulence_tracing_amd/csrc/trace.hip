@@ -1633,6 +1633,16 @@ BatchLayout batch_layout(int32_t nitems, int64_t nchunks) {
     return L;
 }
 
+// Rays a chunk has at most: whole blocks of 256, so that a block's threads all
+// have a ray but in an item's last one, and no more than the largest item, so that
+// no block is launched for rays that no item has (the blocks are per chunk).
+int32_t chunk_rays(const tt_batch_item *items, int32_t nitems, int32_t chunk) {
+    int64_t most = 1;
+    for (int i = 0; i < nitems; ++i) most = std::max(most, items[i].n);
+    chunk = std::min(chunk, 1 << 30);
+    return (int32_t)(256 * std::min(tt::ceil_div((int64_t)chunk, (int64_t)256), tt::ceil_div(most, (int64_t)256)));
+}
+
 int64_t count_chunks(const tt_batch_item *items, int32_t nitems, int32_t chunk) {
     int64_t c = 0;
     for (int i = 0; i < nitems; ++i) c += tt::ceil_div(items[i].n, (int64_t)chunk);
@@ -1642,6 +1652,7 @@ int64_t count_chunks(const tt_batch_item *items, int32_t nitems, int32_t chunk) 
 
 extern "C" int tt_batch_workspace_bytes(const tt_batch_item *items, int32_t nitems, int32_t chunk, size_t *bytes) {
     TT_REQUIRE(items && bytes && nitems >= 1 && chunk >= 1, "tt_batch_workspace_bytes: bad arguments");
+    chunk = chunk_rays(items, nitems, chunk);
     *bytes = batch_layout(nitems, count_chunks(items, nitems, chunk)).total;
     return TT_OK;
 }
@@ -1653,6 +1664,7 @@ extern "C" int tt_batch_prepare(const tt_batch_item *items, int32_t nitems, doub
     const double mm = 1.0 / h;
     const int m = (int)llround(mm);
     TT_REQUIRE(m >= 1 && m <= 64 && fabs(mm - m) < 1e-9, "tt_batch_prepare: h must be 1/m cells with 1 <= m <= 64");
+    chunk = chunk_rays(items, nitems, chunk);
     const int64_t nchunks = count_chunks(items, nitems, chunk);
     TT_REQUIRE(nchunks >= 1 && nchunks < (1ll << 31), "tt_batch_prepare: no rays or too many chunks");
     const BatchLayout L = batch_layout(nitems, nchunks);
@@ -1731,15 +1743,22 @@ extern "C" int tt_batch_trace(void *workspace, const tt_batch_info *info, const 
                "tt_batch_trace: LDS limit");
     }
     const int per = (int)tt::ceil_div(info->chunk, tune->block);
-    const dim3 grid((unsigned)(tt::ceil_div(info->nchunks, kXcds) * kXcds * per));
     const char *w = static_cast<const char *>(workspace);
     const BatchLayout L = batch_layout(info->nitems, info->nchunks);
     hipStream_t st = tt::as_stream(stream);
     const TraceArgs *items = reinterpret_cast<const TraceArgs *>(w + L.items);
     const int32_t *citem = reinterpret_cast<const int32_t *>(w + L.citem);
     const int64_t *cstart = reinterpret_cast<const int64_t *>(w + L.cstart);
-    hipLaunchKernelGGL(kern, grid, dim3(tune->block), lds, st, items, citem, cstart, info->nchunks, info->chunk, per);
-    TT_LAUNCH_CHECK("tt_batch_trace launch");
+    // a launch has fewer than 2^32 threads: as many whole rounds of the XCDs as that takes
+    const int64_t round = (int64_t)kXcds * per * tune->block;
+    const int64_t most = 0xffffffffll / round * kXcds;
+    for (int64_t first = 0; first < info->nchunks; first += most) {
+        const int count = (int)std::min(most, info->nchunks - first);
+        const dim3 grid((unsigned)(tt::ceil_div(count, kXcds) * kXcds * per));
+        hipLaunchKernelGGL(kern, grid, dim3(tune->block), lds, st, items, citem + first, cstart + first, count,
+                           info->chunk, per);
+        TT_LAUNCH_CHECK("tt_batch_trace launch");
+    }
     // the rays handed over (items with a status array), after the whole z-march
     hipLaunchKernelGGL(trace_time_batch_kernel, dim3((unsigned)info->nchunks), dim3(256), 0, st, items, citem, cstart,
                        info->chunk);
