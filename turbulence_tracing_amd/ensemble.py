@@ -154,7 +154,9 @@ class Ensemble:
 
     # ------------------------------------------------------------ tuning
     def signature(self):
-        return {"members": [(m.n, m.n_rays) for m in self.members], "h": self.h}
+        # "launch" names the batched trace's launch that the candidates were timed
+        # on: saved winners of an earlier one (a queue of chunks) are not taken
+        return {"members": [(m.n, m.n_rays) for m in self.members], "h": self.h, "launch": "blocks of chunks"}
 
     def autotune(self, tuner=None, candidates=None, force=False):
         """Pick the trace launch shape, variant, chunk and ordering brick
