@@ -29,3 +29,13 @@ def test_blocks_resident_on_a_cu(tmp_path):
         best = max(units // u for u in range(1, units + 1) if units // u <= blocks)
         assert fit == best, (blocks, lds)
     assert [units // (lds // 1280) for _, lds in got[:12]] == list(range(1, 13))
+
+
+def test_blocks_beyond_one_axis_of_a_grid(tmp_path):
+    cases = [(b, t) for t in (64, 256, 512) for top in [(1 << 32) // t]
+             for b in (1, 2, top - 2, top - 1, top, top + 1, 2 * top - 2, 2 * top, 5 * top + 3, 1 << 30)]
+    body = "".join(f'{{ auto g = tt::spread({b}ll, {t}); std::printf("%u %u\\n", g.x, g.y); }}\n' for b, t in cases)
+    for (b, t), (x, y) in zip(cases, run(tmp_path, body), strict=True):
+        assert x * t < 1 << 32 and 1 <= y <= 65535
+        assert b <= x * y < b + y  # every block, and fewer spare ones than rows
+        assert (y == 1) == (b * t < 1 << 32)

@@ -17,6 +17,7 @@
 // memory directly.
 #include <algorithm>
 
+#include "launch_shape.h"
 #include "tt_internal.h"
 
 #pragma clang fp contract(off)
@@ -127,7 +128,7 @@ __device__ __forceinline__ int wave_max(int v) {
 __global__ __launch_bounds__(kDetBlock) void detect_kernel(DetArgs a) {
     __shared__ uint32_t lds[kLdsBins];
     __shared__ int win[4];  // bx0, bx1, by0, by1 of this block's hits
-    const int64_t i = (int64_t)blockIdx.x * kDetBlock + threadIdx.x;
+    const int64_t i = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kDetBlock + threadIdx.x;
     const bool live = i < a.n;
     double x0 = 0.0, th0 = 0.0, y0 = 0.0, ph0 = 0.0, phase = 0.0;
     if (live) {
@@ -319,8 +320,8 @@ extern "C" int tt_detect(const tt_detector *dets, int32_t ndet, const double *rf
     a.ld = ld;
     a.n = n;
     a.phase = phase;
-    hipLaunchKernelGGL(detect_kernel, dim3((unsigned)tt::ceil_div(n, (int64_t)kDetBlock)), dim3(kDetBlock), 0,
-                       tt::as_stream(stream), a);
+    const tt::Blocks b = tt::spread(tt::ceil_div(n, (int64_t)kDetBlock), kDetBlock);
+    hipLaunchKernelGGL(detect_kernel, dim3(b.x, b.y), dim3(kDetBlock), 0, tt::as_stream(stream), a);
     TT_LAUNCH_CHECK("tt_detect launch");
     return TT_OK;
 }

@@ -1,7 +1,21 @@
 // Arithmetic of launch shapes, apart from the kernels (plain C++).
 #pragma once
+#include <cstdint>
 
 namespace tt {
+
+// A launch holds fewer than 2^32 threads along each axis of its grid: of one that
+// asks for more, blocks go missing without an error.  More blocks than that go in
+// rows of equal length; block (x, y) takes part
+// y * gridDim.x + x, if there is one (some of the last row's may have none).
+struct Blocks {
+    uint32_t x, y;
+};
+constexpr Blocks spread(int64_t blocks, int threads) {
+    const int64_t most = 0xffffffffll / threads;
+    const int64_t rows = (blocks + most - 1) / most;
+    return rows <= 1 ? Blocks{(uint32_t)blocks, 1u} : Blocks{(uint32_t)((blocks + rows - 1) / rows), (uint32_t)rows};
+}
 
 // LDS of a CU, and the unit in which a block's share of it is given out.
 constexpr int kLdsBytes = 160 * 1024, kLdsGranule = 1280;
