@@ -20,6 +20,7 @@
 #include <cmath>
 #include <vector>
 
+#include "launch_shape.h"
 #include "tt_internal.h"
 
 namespace {
@@ -777,10 +778,11 @@ __global__ __launch_bounds__(kAnyThreads) __attribute__((amdgpu_waves_per_eu(6, 
     for (int j = threadIdx.x; j < n; j += kAnyThreads) tw[j] = a.tw[j];
     // pencils: columns (elements `step` apart from `base`) or rows
     constexpr bool kRows = MODE == kPassX || MODE == kFwdX;
-    const int64_t first = (int64_t)blockIdx.x * PB;
+    const int64_t first = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * PB;
     const int64_t plane = (int64_t)a.nxh * a.ny;
     const int p0 = threadIdx.x & (PB - 1), j0 = threadIdx.x >> lb, dj = kAnyThreads >> lb;
     const int64_t count = kRows ? (int64_t)a.ny * a.nz : MODE == kPassY ? (int64_t)a.nxh * a.nz : plane;
+    if (first >= count) return;  // a spare block of the last row (tt::spread)
     const float in_ = 1.0f / (float)n;
     int kx = 0, ky = 0;
     int64_t base = 0, step = 0;
@@ -1027,9 +1029,8 @@ void launch_pass(tt_fft_plan plan, int ax, hipStream_t st, PassArgs a, size_t ex
     const int64_t count = kRows ? (int64_t)plan->ny * plan->nz : (int64_t)plan->nxh * (MODE == kPassY ? plan->nz : plan->ny);
     if (!fixed_length(n)) {
         a.lb = pencils_any(n, extra);
-        hipLaunchKernelGGL(fft_any_kernel<MODE>, dim3((unsigned)tt::ceil_div(count, (int64_t)1 << a.lb)),
-                           dim3(kAnyThreads),
-                           smem_any(n, a.lb) + extra, st, a);
+        const tt::Blocks b = tt::spread(tt::ceil_div(count, (int64_t)1 << a.lb), kAnyThreads);
+        hipLaunchKernelGGL(fft_any_kernel<MODE>, dim3(b.x, b.y), dim3(kAnyThreads), smem_any(n, a.lb) + extra, st, a);
         return;
     }
     const int64_t B = kBatch / n;
