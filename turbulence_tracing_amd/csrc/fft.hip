@@ -470,7 +470,7 @@ __device__ __forceinline__ Bins bins_of(const PassArgs &a, int jx, int jy, int j
 // 512 blocks: two a CU, which is what the tile loop's registers let run (1024:
 // 142 and 148; a tile a block 144 and 151).
 constexpr int kPowBlocks = 512;
-extern __shared__ float2 smem[];
+extern __shared__ __attribute__((aligned(16))) float2 smem[];
 struct Histogram {
     // places in LDS, in eight and in four bytes (kept as numbers: through
     // pointers held here the adds become flat ones): the block's sums and
@@ -721,6 +721,7 @@ __device__ __forceinline__ void any_pass_prime(const float2 *in, float2 *out, in
             float2 x[kP];  // at()
             const char *px = in0 + erow + (((uint32_t)p0 * 8u) ^ (e8 & swz));
             if (lb > 0) {
+                static_assert(__alignof__(smem) % sizeof(float4) == 0, "two pencils are read at once");
                 const float4 xx = *reinterpret_cast<const float4 *>(px);
                 x[0] = make_float2(xx.x, xx.y);
                 x[1] = make_float2(xx.z, xx.w);
