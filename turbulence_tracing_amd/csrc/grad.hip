@@ -37,6 +37,18 @@ __device__ __forceinline__ T grad1(T sm, T s0, T sp, int i, int n, T c) {
     return (sp - sm) * c;
 }
 
+// the node of stencil value s and gradient (gx, gy, gz), streamed past the caches
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ __forceinline__ void write_node(const GradArgs<T> &a, int ix, int iy, int iz, T s, T gx, T gy, T gz) {
+    const double r = a.alpha + (double)s;
+    const double q = 1.0 - r;
+    // n - 1 = -r / (1 + sqrt(1 - r)), evaluated without cancellation
+    const double eta = q > 0.0 ? -r / (1.0 + sqrt(q)) : -1.0;
+    const f32x4 v = {(float)gx, (float)gy, (float)gz, (float)(eta * (double)a.phase_scale)};
+    __builtin_nontemporal_store(v, reinterpret_cast<f32x4 *>(a.out + ((int64_t)iz * a.ny + iy) * a.nx + ix));
+}
+
 // One pass bound by HBM.  A block owns a tile of the plane of x and a second
 // axis b (z if the input is contiguous along z, else y) and marches along the
 // third axis c.  Each plane of the tile, with a halo of one node, is read once
@@ -48,11 +60,10 @@ __device__ __forceinline__ T grad1(T sm, T s0, T sp, int i, int n, T c) {
 // four fifths of the bytes (fp32 input).
 // Measured: 512^3 fp32 x-fastest 527 us (5.1 TB/s; 915 as a column walk that
 // met its x and y neighbours in L1), 1024^3 3.93 ms (7.28), 201^3 fp64
-// z-fastest 58 us (490 with strided lanes), 512^3 fp64 z-fastest 0.73 ms
+// z-fastest 56 us (490 with strided lanes), 512^3 fp64 z-fastest 0.73 ms
 // (7.13).  With eta left out 516 us: the fp64 root and quotient are hidden.
 // Tiles of 64 x 16 where the lanes run along x (32 x 32: 552 us); 32 x 32 where
 // they run along b, so both axes move at least 128 bytes at a time.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <typename T, int TX, bool BZ, bool FASTX>
 __global__ __launch_bounds__(256) void grad_kernel(GradArgs<T> a) {
@@ -122,22 +133,42 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs<T> a) {
             const T gx = grad1(l[o - 1], s, l[o + 1], ix, a.nx, a.cx);
             const T gb = grad1(l[o - P], s, l[o + P], ib, nb, BZ ? a.cz : a.cy);
             const T gc = grad1(cm[j], s, cp, c, nc, BZ ? a.cy : a.cz);
-            f32x4 ov;
-            ov.x = (float)gx;
-            ov.y = (float)(BZ ? gc : gb);
-            ov.z = (float)(BZ ? gb : gc);
-            const double r = a.alpha + (double)s;
-            const double q = 1.0 - r;
-            const double eta = q > 0.0 ? -r / (1.0 + sqrt(q)) : -1.0;
-            ov.w = (float)(eta * (double)a.phase_scale);
-            if (ix < a.nx && ib < nb) {
-                const int64_t i = BZ ? ((int64_t)ib * a.ny + c) * a.nx + ix : ((int64_t)c * a.ny + ib) * a.nx + ix;
-                __builtin_nontemporal_store(ov, reinterpret_cast<f32x4 *>(a.out + i));
-            }
+            if (ix < a.nx && ib < nb) write_node(a, ix, BZ ? c : ib, BZ ? ib : c, s, gx, BZ ? gc : gb, BZ ? gb : gc);
             cm[j] = s;
             s0[j] = cp;
         }
         cur = nxt;
+    }
+}
+
+// Grids of a few planes along b: those tiles would be mostly empty.  A thread walks
+// one (x, y) column, carrying the z neighbours in registers and meeting those in x
+// and y, which its block's 64 x 4 columns read together, in L1.
+template <typename T>
+__global__ __launch_bounds__(256) void grad_columns_kernel(GradArgs<T> a) {
+    const int ix = (int)blockIdx.x * 64 + threadIdx.x % 64, iy = (int)blockIdx.y * 4 + threadIdx.x / 64;
+    if (ix >= a.nx || iy >= a.ny) return;
+    const int z0 = (int)blockIdx.z * a.run, z1 = min(z0 + a.run, a.nz);
+    T beta = a.beta;
+    if (a.sumsq) beta = (T)((double)beta / sqrt(*a.sumsq / a.count));
+    const auto at = [&](int x, int y, int z) {
+        const T v = a.f[x * a.sx + y * a.sy + z * a.sz] * beta;
+        return v < a.clipv ? v : a.clipv;
+    };
+    T zm = z0 > 0 ? at(ix, iy, z0 - 1) : (T)0;
+    T s0 = at(ix, iy, z0);
+    for (int iz = z0; iz < z1; ++iz) {
+        __builtin_amdgcn_s_setprio(1);  // the plane's loads leave before other waves' arithmetic
+        const T zp = iz < a.nz - 1 ? at(ix, iy, iz + 1) : s0;
+        const T xm = ix > 0 ? at(ix - 1, iy, iz) : s0;
+        const T xp = ix < a.nx - 1 ? at(ix + 1, iy, iz) : s0;
+        const T ym = iy > 0 ? at(ix, iy - 1, iz) : s0;
+        const T yp = iy < a.ny - 1 ? at(ix, iy + 1, iz) : s0;
+        __builtin_amdgcn_s_setprio(0);
+        write_node(a, ix, iy, iz, s0, grad1(xm, s0, xp, ix, a.nx, a.cx), grad1(ym, s0, yp, iy, a.ny, a.cy),
+                   grad1(zm, s0, zp, iz, a.nz, a.cz));
+        zm = s0;
+        s0 = zp;
     }
 }
 
@@ -211,14 +242,30 @@ int launch(const void *field, int64_t sx, int64_t sy, int64_t sz, const tt_grid 
     const auto mag = [](int64_t v) { return v < 0 ? -v : v; };
     const bool bz = mag(sz) < mag(sy) && mag(sz) < mag(sx), fx = !bz && mag(sx) <= mag(sy);
     const int tx = fx ? 64 : 32, tb = 1024 / tx;
-    const int nb = bz ? g->nz : g->ny, nc = bz ? g->ny : g->nz;
-    const int64_t tiles = (int64_t)tt::ceil_div(g->nx, tx) * tt::ceil_div(nb, tb);
-    // Runs of 32 planes where that still gives 2048 blocks (8 per CU), shorter
-    // ones on smaller grids: 48^3 fp64 8.9 us with runs of 2, 11.7 with 4 (64
-    // planes at 512^3: 544 us).
-    a.run = 32;
-    while (a.run > 2 && tiles * tt::ceil_div(nc, a.run) < 2048) a.run /= 2;
-    const dim3 grid((unsigned)tt::ceil_div(g->nx, tx), (unsigned)tt::ceil_div(nb, tb), (unsigned)tt::ceil_div(nc, a.run));
+    const int nb = bz ? g->nz : g->ny;
+    // The longest runs, up to `longest`, that still give `enough` blocks.
+    const auto shape = [&](int bx, int bb, int nbb, int nc, int longest, int enough) {
+        const int64_t tiles = tt::ceil_div(g->nx, bx) * tt::ceil_div(nbb, bb);
+        a.run = longest;
+        while (a.run > 2 && tiles * tt::ceil_div(nc, a.run) < enough) a.run /= 2;
+        return dim3((unsigned)tt::ceil_div(g->nx, bx), (unsigned)tt::ceil_div(nbb, bb),
+                    (unsigned)tt::ceil_div(nc, a.run));
+    };
+    // On a few planes along b most of a tile is empty: 1024 x 1024 x 3 fp32 13 us by
+    // columns and 45 by tiles (z fastest, x next), x 6 32 and 46, x 8 76 and 47; with
+    // x fastest 1024 x 8 x 1024 fp64 46 and 50.  Columns of an input with z fastest
+    // and x slowest lie far apart: 1024 x 1024 x 3 41 and 46, x 4 53 and 45.
+    if (nb <= (fx ? 8 : bz && mag(sx) > mag(sy) ? 3 : 6)) {
+        const dim3 grid = shape(64, 4, g->ny, g->nz, 16, bz ? 1 : 2048);
+        hipLaunchKernelGGL(grad_columns_kernel<T>, grid, dim3(256), 0, st, a);
+        TT_LAUNCH_CHECK("tt_grad_stencil launch");
+        return TT_OK;
+    }
+    // Runs of 32 planes (64 at 512^3: 544 us); on smaller grids shorter ones, which
+    // give more blocks and read their two planes of halo more often: about five
+    // blocks a CU, four where lanes run along x, and half of that in fp64.
+    const int enough = !fx ? 1280 : sizeof(T) == 4 ? 1024 : 512;
+    const dim3 grid = shape(tx, tb, nb, bz ? g->ny : g->nz, 32, enough);
     if (bz)
         hipLaunchKernelGGL((grad_kernel<T, 32, true, false>), grid, dim3(256), 0, st, a);
     else if (fx)
