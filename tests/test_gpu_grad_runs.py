@@ -12,8 +12,8 @@ pytestmark = pytest.mark.gpu
 # Runs by order (x-, y- / z-contiguous) in fp32 and fp64: 8 / 4 and 16 / 4; 16 / 16
 # and 32 / 16; 32 / 32 and 32 / 32
 DEEP = [(201, 201, 203), (260, 250, 270), (400, 330, 420)]
-# up to 3, 6 or 8 planes along y or z (by order), and one more
-THIN = [(150, 40, 4), (40, 150, 3), (40, 150, 6), (40, 150, 7), (33, 8, 70), (300, 5, 33), (130, 7, 2), (65, 9, 17),
+# up to 4, 6 or 8 planes along y or z (by order), and one more
+THIN = [(150, 40, 4), (40, 150, 5), (40, 150, 6), (40, 150, 7), (33, 8, 70), (300, 5, 33), (130, 7, 2), (65, 9, 17),
         (2, 2, 700), (700, 2, 2), (3, 700, 3), (64, 4, 64)]
 
 

@@ -254,8 +254,8 @@ int launch(const void *field, int64_t sx, int64_t sy, int64_t sz, const tt_grid 
     // On a few planes along b most of a tile is empty: 1024 x 1024 x 3 fp32 13 us by
     // columns and 45 by tiles (z fastest, x next), x 6 32 and 46, x 8 76 and 47; with
     // x fastest 1024 x 8 x 1024 fp64 46 and 50.  Columns of an input with z fastest
-    // and x slowest lie far apart: 1024 x 1024 x 3 41 and 46, x 4 53 and 45.
-    if (nb <= (fx ? 8 : bz && mag(sx) > mag(sy) ? 3 : 6)) {
+    // and x slowest lie far apart: x 3 41 and 46, x 4 53 and 45 (300 x 300 x 4 8.2 and 10.4).
+    if (nb <= (fx ? 8 : bz && mag(sx) > mag(sy) ? 4 : 6)) {
         const dim3 grid = shape(64, 4, g->ny, g->nz, 16, bz ? 1 : 2048);
         hipLaunchKernelGGL(grad_columns_kernel<T>, grid, dim3(256), 0, st, a);
         TT_LAUNCH_CHECK("tt_grad_stencil launch");
