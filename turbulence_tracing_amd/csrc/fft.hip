@@ -640,8 +640,8 @@ __global__ __launch_bounds__(kThreads) void fft_pass_kernel(PassArgs a) {
 }
 
 // ---------------------------------------------------------------------
-// Any other length.  A block takes PB pencils (a power of two, 16 up to 600
-// points) in LDS as [element][pencil], two copies of them, and each Stockham
+// Any other length.  A block takes PB pencils (a power of two, 16 up to 309
+// points, more of short ones) in LDS as [element][pencil], two copies of them, and each Stockham
 // pass goes from one to the other: one barrier a pass, and any number of
 // butterflies a thread.  Lanes run over pencils first, so neighbouring lanes
 // share a butterfly: its twiddles are LDS broadcasts, and the columns of passes
@@ -779,7 +779,13 @@ __global__ __launch_bounds__(kAnyThreads) __attribute__((amdgpu_waves_per_eu(6, 
     for (int j = threadIdx.x; j < n; j += kAnyThreads) tw[j] = a.tw[j];
     // pencils: columns (elements `step` apart from `base`) or rows
     constexpr bool kRows = MODE == kPassX || MODE == kFwdX;
-    const int64_t first = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * PB;
+    // Neighbouring columns share the lines that their elements lie in: blocks of
+    // neighbouring columns go to one XCD, whose L2 then holds a line for all of
+    // them (a block of 4 moves 32 bytes of each).  Fields of 256 x 1280 x 256 1417 ->
+    // 1000 us, 128 x 4096 x 128 1840 -> 1354, 320^3 380 -> 343.
+    const int64_t block = kRows || gridDim.y > 1 ? (int64_t)blockIdx.y * gridDim.x + blockIdx.x
+                                                 : tt::xcd_block((int)blockIdx.x, (int)gridDim.x);
+    const int64_t first = block * PB;
     const int64_t plane = (int64_t)a.nxh * a.ny;
     const int p0 = threadIdx.x & (PB - 1), j0 = threadIdx.x >> lb, dj = kAnyThreads >> lb;
     const int64_t count = kRows ? (int64_t)a.ny * a.nz : MODE == kPassY ? (int64_t)a.nxh * a.nz : plane;
@@ -919,9 +925,17 @@ size_t smem_any(int n, int lb) { return (((size_t)2 << lb) + 1) * n * sizeof(flo
 // log2 of the pencils a block takes: 16 while two blocks fit a CU's LDS (up to
 // 309 points), then 8, 4 and 2.  One block of 16 alone on a CU leaves it idle
 // between its passes: 640^3 took 8360 us with 8 pencils against 4350 with 4 (256
-// threads), 320^3 816 with 16 against 465 with 8.
-int pencils_any(int n, size_t extra) {
+// threads), 320^3 816 with 16 against 465 with 8.  Where 16 short pencils would
+// leave most of the 512 threads without an element, more of them, up to 2048
+// elements, as long as that leaves 4 blocks a CU: fields of 2048 x 2048 x 4 684 ->
+// 300 us, 512 x 512 x 12 76 -> 55, 512 x 48 x 512 169 -> 153 (up to 1024 elements:
+// 300, 58 and 169; 32^3 with a quarter of a block a CU 15 -> 19).  At most 256, so
+// that a pencil has two threads.
+constexpr int kMostPencils = 8;
+static_assert(1 << kMostPencils < kAnyThreads, "threads a pencil");
+int pencils_any(int n, int64_t count, size_t extra) {
     int lb = 4;
+    while (lb < kMostPencils && (n << (lb + 1)) <= 2048 && (count >> (lb + 1)) >= 1024) ++lb;
     while (lb > 1 && smem_any(n, lb) + extra > kMaxLds / 2) --lb;
     while (lb > 0 && smem_any(n, lb) + extra > kMaxLds) --lb;
     return lb;
@@ -1029,7 +1043,7 @@ void launch_pass(tt_fft_plan plan, int ax, hipStream_t st, PassArgs a, size_t ex
     constexpr bool kRows = MODE == kPassX || MODE == kFwdX;
     const int64_t count = kRows ? (int64_t)plan->ny * plan->nz : (int64_t)plan->nxh * (MODE == kPassY ? plan->nz : plan->ny);
     if (!fixed_length(n)) {
-        a.lb = pencils_any(n, extra);
+        a.lb = pencils_any(n, count, extra);
         const tt::Blocks b = tt::spread(tt::ceil_div(count, (int64_t)1 << a.lb), kAnyThreads);
         hipLaunchKernelGGL(fft_any_kernel<MODE>, dim3(b.x, b.y), dim3(kAnyThreads), smem_any(n, a.lb) + extra, st, a);
         return;
