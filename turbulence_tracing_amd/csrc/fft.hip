@@ -257,7 +257,12 @@ __device__ __forceinline__ void last_pass(const float2 *buf, const float2 *tw, S
             else
                 dft<R>(v);
 #pragma unroll
-            for (int q = 0; q < R; ++q) store(p, b + NS * q, v[q]);
+            for (int q = 0; q < R; ++q) {
+                if constexpr (POW)
+                    store(i * R + q, v[q]);
+                else
+                    store(p, b + NS * q, v[q]);
+            }
         }
     }
 }
@@ -282,7 +287,7 @@ constexpr int outputs_of() {
     else
         return outputs_of<N, NS * R>();
 }
-// f(p, j) over them, in the order the last pass stores them
+// f(i, p, j) over them, i as the last pass numbers them
 template <int N, bool PFAST, int NS = 1, class F>
 __device__ __forceinline__ void each_output(F f) {
     constexpr int R = radix_at<N, NS>();
@@ -295,7 +300,7 @@ __device__ __forceinline__ void each_output(F f) {
                 int p, b;
                 split_bf<B, NS, PFAST>(beta, p, b);
 #pragma unroll
-                for (int q = 0; q < R; ++q) f(p, b + NS * q);
+                for (int q = 0; q < R; ++q) f(i * R + q, p, b + NS * q);
             }
         }
     } else {
@@ -303,7 +308,8 @@ __device__ __forceinline__ void each_output(F f) {
     }
 }
 
-// the whole transform of the block's B pencils: load(p, j) -> store(p, j, v)
+// the whole transform of the block's B pencils: load(p, j) -> store(p, j, v), or
+// (POW) store(i, v) for the thread's i-th output, each_output's numbers
 template <int N, bool PFAST, bool POW = false, class Load, class Store>
 __device__ __forceinline__ void fft_pow2(float2 *buf, const float2 *tw, Load load, Store store) {
     first_pass<N, PFAST>(buf, load);
@@ -468,7 +474,9 @@ __device__ __forceinline__ Bins bins_of(const PassArgs &a, int jx, int jy, int j
 // the block's own bins, a tile a block, and a double quotient, root and integer
 // remainders an element; 134 and 140 now, 512^3 983 and 1214 -> 888 and 910.
 // 512 blocks: two a CU, which is what the tile loop's registers let run (1024:
-// 142 and 148; a tile a block 144 and 151).
+// 142 and 148; a tile a block 144 and 151).  Two waves a SIMD are asked for: 384
+// points, whose 33 outputs a thread take the most registers, would run one (384^3
+// 666 and 730 us, with the powers in scratch; 540 and 564 with neither).
 constexpr int kPowBlocks = 512;
 extern __shared__ __attribute__((aligned(16))) float2 smem[];
 struct Histogram {
@@ -551,7 +559,7 @@ __device__ __forceinline__ void block_sum(double v, double *out) {
 
 // The fixed lengths: NF points a pencil, kBatch / NF pencils a block.
 template <int MODE, int NF>
-__global__ __launch_bounds__(kThreads) void fft_pass_kernel(PassArgs a) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MODE == kPowZ ? 2 : 1))) void fft_pass_kernel(PassArgs a) {
     constexpr int BF = kBatch / NF;
     float2 *buf = smem;
     float2 *tw = smem + BF * (NF + 1);
@@ -569,14 +577,12 @@ __global__ __launch_bounds__(kThreads) void fft_pass_kernel(PassArgs a) {
         H.clear_own(kThreads);
         for (int64_t first = (int64_t)blockIdx.x * BF; first < plane; first += (int64_t)gridDim.x * BF) {
             float power[outputs_of<NF>()];
-            int n = 0;
             fft_pow2<NF, true, true>(
                 buf, tw,
                 [&](int p, int j) { return first + p < plane ? a.spec[j * plane + first + p] : make_float2(0.f, 0.f); },
-                [&](int, int, float2 v) { power[n++] = fmaf(v.x, v.x, v.y * v.y); });
+                [&](int i, float2 v) { power[i] = fmaf(v.x, v.x, v.y * v.y); });
             __syncthreads();
-            n = 0;
-            each_output<NF, true>([&](int p, int j) { pw[j * BF + p] = power[n++]; });
+            each_output<NF, true>([&](int i, int p, int j) { pw[j * BF + p] = power[i]; });
             H.clear_copies(kThreads);
             __syncthreads();
 #pragma unroll 1
