@@ -112,6 +112,25 @@ __device__ __forceinline__ int wave_max(int v) {
     return v;
 }
 
+// A ray carried to a detector: where it meets it and its bin there (bx < 0: none)
+struct Hit {
+    double x;
+    int bx, by;
+};
+__device__ __forceinline__ Hit hit(const DetDev &d, bool live, double x, double th, double y, double ph) {
+    Hit h{0.0, -1, -1};
+    if (live && apply_train(d, x, th, y, ph)) {
+        h.bx = bin_of(x, d.xmin, d.xmax, d.xstep, d.xinv, d.nbx);
+        h.by = bin_of(y, d.ymin, d.ymax, d.ystep, d.yinv, d.nby);
+    }
+    h.x = x;
+    if (h.by < 0) h.bx = -1;
+    return h;
+}
+__device__ __forceinline__ float weight(const DetDev &d, double phase, double x) {
+    return (float)(1.0 + cos(phase - d.tilt_k * x));
+}
+
 // A block takes its rays through each detector in turn: the bin window of its
 // hits (wave reductions, then 4 LDS atomics per wave), a private LDS copy of
 // that window when it holds at most kLdsBins bins, then the non-zero bins
@@ -147,22 +166,15 @@ __global__ __launch_bounds__(kDetBlock) void detect_kernel(DetArgs a) {
         }
     };
     clear_window();
-    double xd = 0.0;       // at the detector
-    int bx = -1, by = -1;  // its bin; bx < 0: none
+    Hit h{0.0, -1, -1};
     int wx0 = 0, wy0 = 0, ww = 0;
     int64_t area = 0;
     for (int k = 0; k < a.ndet; ++k) {
         const DetDev &d = a.d[k];
         lds_barrier();  // win is cleared; the previous detector's LDS flush reads are done
         if (!d.again) {
-            double x = x0, th = th0, y = y0, ph = ph0;
-            bx = by = -1;
-            if (live && apply_train(d, x, th, y, ph)) {
-                bx = bin_of(x, d.xmin, d.xmax, d.xstep, d.xinv, d.nbx);
-                by = bin_of(y, d.ymin, d.ymax, d.ystep, d.yinv, d.nby);
-            }
-            xd = x;
-            if (by < 0) bx = -1;
+            h = hit(d, live, x0, th0, y0, ph0);
+            const int bx = h.bx, by = h.by;
             const int lx0 = wave_min(bx >= 0 ? bx : 0x7fffffff), lx1 = wave_max(bx);
             const int ly0 = wave_min(bx >= 0 ? by : 0x7fffffff), ly1 = wave_max(bx >= 0 ? by : -1);
             if ((threadIdx.x & 63) == 0 && lx1 >= 0) {
@@ -177,8 +189,9 @@ __global__ __launch_bounds__(kDetBlock) void detect_kernel(DetArgs a) {
             ww = win[1] - wx0 + 1;
             area = win[1] >= wx0 ? (int64_t)ww * (win[3] - wy0 + 1) : 0;
         }
+        const int bx = h.bx, by = h.by;
         float w = 1.0f;
-        if (d.mode == 1 && bx >= 0) w = (float)(1.0 + cos(phase - d.tilt_k * xd));
+        if (d.mode == 1 && bx >= 0) w = weight(d, phase, h.x);
         if (area > 0 && area <= kLdsBins) {
             for (int j = threadIdx.x; j < area; j += kDetBlock) lds[j] = 0u;
             lds_barrier();
@@ -222,6 +235,57 @@ __global__ __launch_bounds__(256) void optics_kernel(DetDev d, const double *rin
     rout[ldo + i] = ok ? th : nanv;
     rout[2 * ldo + i] = ok ? y : nanv;
     rout[3 * ldo + i] = ok ? ph : nanv;
+}
+
+// Many rays on few bins: a block keeps the histograms of all detectors in LDS, takes
+// rays in strides of the grid and adds each bin to memory once.  In detect_kernel
+// every 512 rays add their window's bins; those of rays in launch order are the
+// whole detector, and the adds wait for each other at its few addresses.
+// 1e7 rays in launch order on one detector of 16^2 150 us (543 by windows; 330 with
+// 1024 rays a block there), 128^2 175 (307, 284), three of 64^2 318 (988, 685); sorted
+// 135, 171 and 272 (191, 198 and 562 with 1024 rays a block).
+// From kWholeRays rays a bin on: with fewer a block's own bins outweigh its rays
+// (1e6 rays on 64^2 30 us sorted and 34 in launch order, 21 and 49 by windows; on 90^2
+// 55 and 57, 21 and 50).  Four blocks a CU as far as LDS lets (two: 10% slower).
+constexpr int kWholeBins = 16384;  // of a launch's detectors: 64 KB
+constexpr int kWholeRays = 200;
+extern __shared__ uint32_t whole[];
+__global__ __launch_bounds__(kDetBlock) void detect_whole_kernel(DetArgs a, int bins) {
+    for (int j = threadIdx.x; j < bins; j += kDetBlock) whole[j] = 0u;
+    lds_barrier();
+    for (int64_t i = (int64_t)blockIdx.x * kDetBlock + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * kDetBlock) {
+        const double x = a.rf[i], th = a.rf[a.ld + i], y = a.rf[2 * a.ld + i], ph = a.rf[3 * a.ld + i];
+        const double phase = a.phase ? a.phase[i] : 0.0;
+        Hit h{0.0, -1, -1};
+        int first = 0;
+        for (int k = 0; k < a.ndet; ++k) {
+            const DetDev &d = a.d[k];
+            if (!d.again) h = hit(d, true, x, th, y, ph);
+            if (h.bx >= 0) {
+                const int q = first + h.by * d.nbx + h.bx;
+                if (d.mode == 1)
+                    atomicAdd(reinterpret_cast<float *>(&whole[q]), weight(d, phase, h.x));
+                else
+                    atomicAdd(&whole[q], 1u);
+            }
+            first += d.nbx * d.nby;
+        }
+    }
+    lds_barrier();
+    int first = 0;
+    for (int k = 0; k < a.ndet; ++k) {
+        const DetDev &d = a.d[k];
+        const int n = d.nbx * d.nby;
+        for (int j = threadIdx.x; j < n; j += kDetBlock) {
+            const uint32_t v = whole[first + j];
+            if (v == 0u) continue;
+            if (d.mode == 1)
+                atomicAdd(&d.wsum[j], __uint_as_float(v));
+            else
+                atomicAdd(&d.counts[j], v);
+        }
+        first += n;
+    }
 }
 
 int fill_train(const tt_train *t, DetDev &d) {
@@ -320,6 +384,30 @@ extern "C" int tt_detect(const tt_detector *dets, int32_t ndet, const double *rf
     a.ld = ld;
     a.n = n;
     a.phase = phase;
+    // groups of detectors that detect_whole_kernel takes at once, if it takes them all
+    int group[TT_MAX_DETECTORS], count[TT_MAX_DETECTORS], groups = 0;
+    for (int k = 0; k < ndet && groups >= 0; ++k) {
+        const int64_t bins = (int64_t)a.d[k].nbx * a.d[k].nby;
+        const bool more = groups > 0 && group[groups - 1] + bins <= kWholeBins;
+        if (!more) group[groups] = count[groups] = 0, ++groups;
+        ++count[groups - 1];
+        if (bins > kWholeBins || n < kWholeRays * (group[groups - 1] += (int)bins)) groups = -1;
+    }
+    if (groups > 0) {
+        for (int g = 0, k = 0; g < groups; k += count[g], ++g) {
+            DetArgs w = a;
+            w.ndet = count[g];
+            std::copy(a.d + k, a.d + k + count[g], w.d);
+            w.d[0].again = 0;
+            // resident at once, each with as many rays as bins to add at least
+            const int64_t blocks = std::min<int64_t>(256 * std::min(4, kWholeBins * 5 / 2 / group[g]),
+                                                     tt::ceil_div(n, (int64_t)std::max(kDetBlock, group[g])));
+            hipLaunchKernelGGL(detect_whole_kernel, dim3((unsigned)blocks), dim3(kDetBlock),
+                               (size_t)group[g] * sizeof(uint32_t), tt::as_stream(stream), w, group[g]);
+            TT_LAUNCH_CHECK("tt_detect launch");
+        }
+        return TT_OK;
+    }
     const tt::Blocks b = tt::spread(tt::ceil_div(n, (int64_t)kDetBlock), kDetBlock);
     hipLaunchKernelGGL(detect_kernel, dim3(b.x, b.y), dim3(kDetBlock), 0, tt::as_stream(stream), a);
     TT_LAUNCH_CHECK("tt_detect launch");
