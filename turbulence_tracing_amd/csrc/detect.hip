@@ -242,8 +242,10 @@ __global__ __launch_bounds__(256) void optics_kernel(DetDev d, const double *rin
 // every 512 rays add their window's bins; those of rays in launch order are the
 // whole detector, and the adds wait for each other at its few addresses.
 // 1e7 rays in launch order on one detector of 16^2 150 us (543 by windows; 330 with
-// 1024 rays a block there), 128^2 175 (307, 284), three of 64^2 318 (988, 685); sorted
-// 135, 171 and 272 (191, 198 and 562 with 1024 rays a block).
+// 1024 rays a block there), 128^2 175 (307, 284), three of 64^2 317 (988, 681), of
+// 90^2 in two launches 364 (1097, 735), of 128^2 in three 562 (967, 844); sorted 134,
+// 172, 273, 327 and 508 (191, 197, 558, 556 and 554 with 1024 rays a block; the last
+// 342 by windows).
 // From kWholeRays rays a bin on: with fewer a block's own bins outweigh its rays
 // (1e6 rays on 64^2 30 us sorted and 34 in launch order, 21 and 49 by windows; on 90^2
 // 55 and 57, 21 and 50).  Four blocks a CU as far as LDS lets (two: 10% slower).
