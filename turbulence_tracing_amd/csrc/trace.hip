@@ -22,6 +22,7 @@
 // Algorithmic traffic (roofline accounting): 4 stages x 8 corners x 16 B =
 // 512 B per ray-step.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "launch_shape.h"
@@ -801,23 +802,33 @@ __device__ __forceinline__ bool march_m2u(const TraceArgs &a, float pxb, float p
             State yn;
             ZP zc = form_of<FORMS>(load_nodes<FORMS>(base, row, off));
             Nodes up = load_nodes<FORMS>(base + step, row, off);
-            // One whole cell from the cache: its lower plane's form zc comes from
-            // the cell before, the upper one's is left in U for the next; the
-            // nodes above that are loaded a cell ahead.  Returns whether another
-            // cell follows.
-            auto cell = [&](ZP &zc, ZP &U) __attribute__((always_inline)) {
-                U = form_of<FORMS>(up);
-                const ZP D = zsub(U, zc);
-                const ZP zq = zstep(zc, 0.25f, D);
-                const ZP zh = zstep(zc, 0.5f, D);
+            auto ask_ahead = [&]() __attribute__((always_inline)) {
                 __builtin_amdgcn_s_setprio(1);
                 const gbytes ahead = base + 2 * step;
                 up = load_nodes<FORMS>(ahead < last ? ahead : last, row, off);
                 __builtin_amdgcn_s_setprio(0);
+            };
+            // One whole cell from the cache: its lower plane's form zc comes from
+            // the cell before, the upper one's is left in U for the next; the
+            // nodes above that are loaded a cell ahead.  Returns whether another
+            // cell follows.  The first cell after an entry (EARLY false) asks for
+            // them once its first step is good: a wave that has just redone a step
+            // is likely to redo the next, and loads for a cell it enters anew are
+            // bandwidth lost (1e6 rays in launch order through 512^3, ne0 = 1e25, 20%
+            // RMS: 43.1 -> 40.9 ms; sorted 7.55 -> 7.40; asked for there in every
+            // cell 38.0 and 7.33, but 1e5 sorted rays through 512^3 541 -> 552 us).
+            auto cell = [&](auto early, ZP &zc, ZP &U) __attribute__((always_inline)) {
+                constexpr bool EARLY = decltype(early)::value;
+                U = form_of<FORMS>(up);
+                const ZP D = zsub(U, zc);
+                const ZP zq = zstep(zc, 0.25f, D);
+                const ZP zh = zstep(zc, 0.5f, D);
+                if (EARLY) ask_ahead();
                 yn = ys;
                 phi = rk4_half_z<TAU>(sx, sy, zc, zq, zh, ox, oy, yn, iWc, far, em);
                 okm = mask_of(far <= kInCell) & mask_of(em <= kNewtonTol) & in;
                 if (__builtin_expect(okm != act, 0)) return false;
+                if (!EARLY) ask_ahead();
                 ledger_first(L, ph, phi, true, 0.f);
                 good &= mask_of(yn.Wd > kWdMin);
                 ys = yn;
@@ -845,8 +856,10 @@ __device__ __forceinline__ bool march_m2u(const TraceArgs &a, float pxb, float p
                 return true;
             };
             ZP zb;
-            while (cell(zc, zb) && cell(zb, zc)) {  // two cells a turn: no copies from U to zc
-            }
+            constexpr std::true_type kEarly{};
+            if (cell(std::false_type{}, zc, zb))
+                while (cell(kEarly, zb, zc) && cell(kEarly, zc, zb)) {  // two cells a turn: no copies from U to zc
+                }
             // the ways out of that loop meet here: hidden from the compiler,
             // which would otherwise give each its own copy of what follows and
             // pay for it with register copies on the loop's common path
