@@ -1327,12 +1327,12 @@ __device__ __forceinline__ double time_speed2(double U) {
     return quad<2, 2, 2, 2>(fma(U, U, quad<B, B, B, B>(n)));
 }
 
-// sum of c_j k_j, j < n
+// sum of c_j k_j, j < n, terms with c_j = 0 among them: a slope that is infinite or
+// NaN makes the sum NaN there too
 __device__ __forceinline__ double time_dot(const double *c, const double *k, int n) {
     double s = 0.0;
 #pragma unroll
-    for (int j = 0; j < n; ++j)
-        if (c[j] != 0.0) s = fma(c[j], k[j], s);
+    for (int j = 0; j < n; ++j) s = fma(c[j], k[j], s);
     return s;
 }
 
@@ -1403,7 +1403,7 @@ __device__ __forceinline__ void trace_time_quad(const TraceArgs &a, int64_t r) {
             // the largest scaled error estimate, over the quad
             const double ex = L.phase ? 0.0 : time_dot(kDPE, kx, 7), eu = time_dot(kDPE, ku, 7);
             const double su = L.phase ? kTimeTol * fmax(1.0, fmax(fabs(U), fabs(Un))) : kTimeTol;
-            double en = fmax(fabs(hh * ex) / (kTimeTol * L.size), fabs(hh * eu) / su);
+            double en = fmax(0.0, fmax(fabs(hh * ex) / (kTimeTol * L.size), fabs(hh * eu) / su));  // 0 if both are NaN
             en = fmax(en, quad<1, 0, 3, 2>(en));
             en = fmax(en, quad<2, 3, 0, 1>(en));
             double fac = 0.9 * pow(fmax(en, 1e-10), -0.2);
