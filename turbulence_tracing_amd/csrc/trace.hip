@@ -100,67 +100,66 @@ __device__ __forceinline__ float path_factor(const State &s, float W, float iW) 
     return __builtin_amdgcn_sqrtf(fmaf(s.U, s.U, fmaf(s.V, s.V, W * W))) * iW;
 }
 
-template <bool VF>
-__device__ __forceinline__ void rhs(const TraceArgs &a, float pxb, float pyb, float Z, const State &s, State &k,
-                                    float &gw, float &vf) {
-    const float4 g = sample(a, fmaf(a.sx, s.qx, pxb), fmaf(a.sy, s.qy, pyb), Z);
-    const float W = 1.0f + s.Wd;
-    const float iW = __builtin_amdgcn_rcpf(W);
-    k.qx = s.U * iW;
-    k.qy = s.V * iW;
-    k.U = g.x * iW;
-    k.V = g.y * iW;
-    k.Wd = g.z * iW;
-    k.tr = -s.Wd * iW;
-    gw = g.w;
-    if (VF) vf = path_factor(s, W, iW);
-}
-
 __device__ __forceinline__ State axpy(const State &y, float c, const State &k) {
     return State{fmaf(c, k.qx, y.qx), fmaf(c, k.qy, y.qy), fmaf(c, k.U, y.U),
                  fmaf(c, k.V, y.V),   fmaf(c, k.Wd, y.Wd), fmaf(c, k.tr, y.tr)};
 }
 
-// one classic RK4 step of size hh from Z; returns the phase increment
-__device__ __forceinline__ float rk4_step(const TraceArgs &a, float pxb, float pyb, float Z, float hh, State &y) {
-    State k1, k2, k3, k4;
-    float p1, p2, p3, p4, vf = 0.f;
-    const float h2 = 0.5f * hh;
-    rhs<false>(a, pxb, pyb, Z, y, k1, p1, vf);
-    rhs<false>(a, pxb, pyb, Z + h2, axpy(y, h2, k1), k2, p2, vf);
-    rhs<true>(a, pxb, pyb, Z + h2, axpy(y, h2, k2), k3, p3, vf);
-    rhs<false>(a, pxb, pyb, Z + hh, axpy(y, hh, k3), k4, p4, vf);
-    const float h6 = hh * (1.0f / 6.0f);
-    y.qx += h6 * (k1.qx + 2.f * (k2.qx + k3.qx) + k4.qx);
-    y.qy += h6 * (k1.qy + 2.f * (k2.qy + k3.qy) + k4.qy);
-    y.U += h6 * (k1.U + 2.f * (k2.U + k3.U) + k4.U);
-    y.V += h6 * (k1.V + 2.f * (k2.V + k3.V) + k4.V);
-    y.Wd += h6 * (k1.Wd + 2.f * (k2.Wd + k3.Wd) + k4.Wd);
-    y.tr += h6 * (k1.tr + 2.f * (k2.tr + k3.tr) + k4.tr);
-    return h6 * (p1 + 2.f * (p2 + p3) + p4) * vf;
+// One classic RK4 step of size hh by gathers; returns the phase integrand
+// Phi |v| / W at the step's start point and, in dph, the step's phase by the RK4
+// weights.  ask(qx, qy, j) asks for the field at a stage's position, j half steps on,
+// as soon as that is known (it takes the field of the stage before the last one),
+// and take() gives the value.  Every rounding is written out, so a ray's bits do not
+// depend on which form of the march its wave took.
+template <class Ask, class Take>
+__device__ __forceinline__ float rk4_gathered(Ask ask, Take take, float hh, State &y, float &dph) {
+#pragma clang fp contract(off)
+    const float h2 = 0.5f * hh, h6 = hh * (1.0f / 6.0f);
+    const auto G1 = ask(y.qx, y.qy, 0);
+    const float W1 = 1.0f + y.Wd, i1 = __builtin_amdgcn_rcpf(W1);
+    const float k1x = y.U * i1, k1y = y.V * i1;
+    const auto G2 = ask(fmaf(h2, k1x, y.qx), fmaf(h2, k1y, y.qy), 1);
+    const float4 g1 = take(G1);
+    const float vf1 = path_factor(y, W1, i1);
+    const float k1U = g1.x * i1, k1V = g1.y * i1, k1D = g1.z * i1;
+    const float U2 = fmaf(h2, k1U, y.U), V2 = fmaf(h2, k1V, y.V), D2 = fmaf(h2, k1D, y.Wd);
+    const float i2 = __builtin_amdgcn_rcpf(1.0f + D2);
+    const float k2x = U2 * i2, k2y = V2 * i2;
+    const auto G3 = ask(fmaf(h2, k2x, y.qx), fmaf(h2, k2y, y.qy), 1);
+    const float4 g2 = take(G2);
+    const float k2U = g2.x * i2, k2V = g2.y * i2, k2D = g2.z * i2;
+    const State y3{0.f, 0.f, fmaf(h2, k2U, y.U), fmaf(h2, k2V, y.V), fmaf(h2, k2D, y.Wd), 0.f};
+    const float W3 = 1.0f + y3.Wd, i3 = __builtin_amdgcn_rcpf(W3);
+    const float k3x = y3.U * i3, k3y = y3.V * i3;
+    const auto G4 = ask(fmaf(hh, k3x, y.qx), fmaf(hh, k3y, y.qy), 2);
+    const float4 g3 = take(G3);
+    const float vf = path_factor(y3, W3, i3);
+    const float U4 = fmaf(hh, g3.x * i3, y.U), V4 = fmaf(hh, g3.y * i3, y.V), D4 = fmaf(hh, g3.z * i3, y.Wd);
+    const float i4 = __builtin_amdgcn_rcpf(1.0f + D4);
+    const float4 g4 = take(G4);
+    const float tr = fmaf(-D4, i4, fmaf(2.f, fmaf(i3, -y3.Wd, -(D2 * i2)), -(y.Wd * i1)));
+    y.tr = fmaf(h6, tr, y.tr);
+    y.qx = fmaf(h6, fmaf(U4, i4, fmaf(2.f, k2x + k3x, k1x)), y.qx);
+    y.qy = fmaf(h6, fmaf(V4, i4, fmaf(2.f, k2y + k3y, k1y)), y.qy);
+    y.U = fmaf(h6, fmaf(g4.x, i4, fmaf(2.f, fmaf(g3.x, i3, k2U), k1U)), y.U);
+    y.V = fmaf(h6, fmaf(g4.y, i4, fmaf(2.f, fmaf(g3.y, i3, k2V), k1V)), y.V);
+    y.Wd = fmaf(h6, fmaf(g4.z, i4, fmaf(2.f, fmaf(g3.z, i3, k2D), k1D)), y.Wd);
+    dph = h6 * (fmaf(2.f, g2.w + g3.w, g1.w) + g4.w) * vf;
+    return g1.w * vf1;
 }
-
-// One classic RK4 step as rk4_step, returning the phase integrand
-// Phi |v| / W at the step's start point and, in dph, the step's phase by the
-// RK4 weights (the h = 1/2 march uses one or the other).
+// from plane Z (cells)
 __device__ __forceinline__ float rk4_step_phi(const TraceArgs &a, float pxb, float pyb, float Z, float hh, State &y,
                                               float &dph) {
-    State k1, k2, k3, k4;
-    float p1, p2, p3, p4, vf1 = 0.f, vf = 0.f, unused;
-    const float h2 = 0.5f * hh;
-    rhs<true>(a, pxb, pyb, Z, y, k1, p1, vf1);
-    rhs<false>(a, pxb, pyb, Z + h2, axpy(y, h2, k1), k2, p2, unused);
-    rhs<true>(a, pxb, pyb, Z + h2, axpy(y, h2, k2), k3, p3, vf);
-    rhs<false>(a, pxb, pyb, Z + hh, axpy(y, hh, k3), k4, p4, unused);
-    const float h6 = hh * (1.0f / 6.0f);
-    y.qx += h6 * (k1.qx + 2.f * (k2.qx + k3.qx) + k4.qx);
-    y.qy += h6 * (k1.qy + 2.f * (k2.qy + k3.qy) + k4.qy);
-    y.U += h6 * (k1.U + 2.f * (k2.U + k3.U) + k4.U);
-    y.V += h6 * (k1.V + 2.f * (k2.V + k3.V) + k4.V);
-    y.Wd += h6 * (k1.Wd + 2.f * (k2.Wd + k3.Wd) + k4.Wd);
-    y.tr += h6 * (k1.tr + 2.f * (k2.tr + k3.tr) + k4.tr);
-    dph = h6 * (p1 + 2.f * (p2 + p3) + p4) * vf;
-    return p1 * vf1;
+    const auto ask = [&](float qx, float qy, int j) {
+        return sample(a, fmaf(a.sx, qx, pxb), fmaf(a.sy, qy, pyb), j == 0 ? Z : j == 1 ? Z + 0.5f * hh : Z + hh);
+    };
+    return rk4_gathered(ask, [](const float4 &g) { return g; }, hh, y, dph);
+}
+// the same, returning the step's phase
+__device__ __forceinline__ float rk4_step(const TraceArgs &a, float pxb, float pyb, float Z, float hh, State &y) {
+    float dph;
+    rk4_step_phi(a, pxb, pyb, Z, hh, y, dph);
+    return dph;
 }
 
 // The phase integrand Phi |v| / W by trilinear gathers at plane Z (cells),
@@ -719,52 +718,16 @@ __device__ __forceinline__ float4 value(const Gather &G) {
     return make_float4(keep(g.x), keep(g.y), keep(g.z), keep(g.w));
 }
 
-// rk4_step_phi of h = 1/2 from step k, with the nodes of a stage asked for as
-// soon as its position is known: that takes the field of the stage before the
-// last one, so two stages' nodes are on their way at a time.  Every rounding is
-// written out: those of rk4_step_phi as the compiler contracts it, so a ray's
-// bits do not depend on which march its wave took.  A redone step was bound by
-// its four round trips to memory one after the other (a wave redoes one in four
-// cells at 1024^3, one in two where the field is strong): 1e7 rays through
-// 1024^3 87.1 -> 83.4 ms, 1.3e6 through 384^3 with ne0 = 1e25, 20% RMS 7.21 ->
-// 6.98, 1e5 through 128^3 140 -> 137 us.  (A copy per parity, with the cell's
-// midpoint gathered along and the first stage from one plane, spills: 1% slower.)
+// rk4_step_phi of h = 1/2 from step k: two stages' nodes are on their way at a time.
+// A redone step was bound by its four round trips to memory one after the other (a
+// wave redoes one in four cells at 1024^3, one in two where the field is strong):
+// 1e7 rays through 1024^3 87.1 -> 83.4 ms, 1.3e6 through 384^3 with ne0 = 1e25, 20%
+// RMS 7.21 -> 6.98, 1e5 through 128^3 140 -> 137 us.  (A copy per parity, with the
+// cell's midpoint gathered along and the first stage from one plane, spills: 1% slower.)
 __device__ __forceinline__ float rk4_step_phi_u(const GatherAt &A, float sx, float sy, float pxb, float pyb, int k,
                                                 State &y, float &dph) {
-#pragma clang fp contract(off)
-    constexpr float hh = 0.5f, h2 = 0.25f, h6 = hh * (1.0f / 6.0f);
-    const auto at = [&](float qx, float qy, int q) { return gather(A, fmaf(sx, qx, pxb), fmaf(sy, qy, pyb), q); };
-    const Gather G1 = at(y.qx, y.qy, 2 * k);
-    const float W1 = 1.0f + y.Wd, i1 = __builtin_amdgcn_rcpf(W1);
-    const float k1x = y.U * i1, k1y = y.V * i1;
-    const Gather G2 = at(fmaf(h2, k1x, y.qx), fmaf(h2, k1y, y.qy), 2 * k + 1);
-    const float4 g1 = value(G1);
-    const float vf1 = path_factor(y, W1, i1);
-    const float k1U = g1.x * i1, k1V = g1.y * i1, k1D = g1.z * i1;
-    const float U2 = fmaf(h2, k1U, y.U), V2 = fmaf(h2, k1V, y.V), D2 = fmaf(h2, k1D, y.Wd);
-    const float i2 = __builtin_amdgcn_rcpf(1.0f + D2);
-    const float k2x = U2 * i2, k2y = V2 * i2;
-    const Gather G3 = at(fmaf(h2, k2x, y.qx), fmaf(h2, k2y, y.qy), 2 * k + 1);
-    const float4 g2 = value(G2);
-    const float k2U = g2.x * i2, k2V = g2.y * i2, k2D = g2.z * i2;
-    const State y3{0.f, 0.f, fmaf(h2, k2U, y.U), fmaf(h2, k2V, y.V), fmaf(h2, k2D, y.Wd), 0.f};
-    const float W3 = 1.0f + y3.Wd, i3 = __builtin_amdgcn_rcpf(W3);
-    const float k3x = y3.U * i3, k3y = y3.V * i3;
-    const Gather G4 = at(fmaf(hh, k3x, y.qx), fmaf(hh, k3y, y.qy), 2 * k + 2);
-    const float4 g3 = value(G3);
-    const float vf = path_factor(y3, W3, i3);
-    const float U4 = fmaf(hh, g3.x * i3, y.U), V4 = fmaf(hh, g3.y * i3, y.V), D4 = fmaf(hh, g3.z * i3, y.Wd);
-    const float i4 = __builtin_amdgcn_rcpf(1.0f + D4);
-    const float4 g4 = value(G4);
-    const float tr = fmaf(-D4, i4, fmaf(2.f, fmaf(i3, -y3.Wd, -(D2 * i2)), -(y.Wd * i1)));
-    y.tr = fmaf(h6, tr, y.tr);
-    y.qx = fmaf(h6, fmaf(U4, i4, fmaf(2.f, k2x + k3x, k1x)), y.qx);
-    y.qy = fmaf(h6, fmaf(V4, i4, fmaf(2.f, k2y + k3y, k1y)), y.qy);
-    y.U = fmaf(h6, fmaf(g4.x, i4, fmaf(2.f, fmaf(g3.x, i3, k2U), k1U)), y.U);
-    y.V = fmaf(h6, fmaf(g4.y, i4, fmaf(2.f, fmaf(g3.y, i3, k2V), k1V)), y.V);
-    y.Wd = fmaf(h6, fmaf(g4.z, i4, fmaf(2.f, fmaf(g3.z, i3, k2D), k1D)), y.Wd);
-    dph = h6 * (fmaf(2.f, g2.w + g3.w, g1.w) + g4.w) * vf;
-    return g1.w * vf1;
+    const auto ask = [&](float qx, float qy, int j) { return gather(A, fmaf(sx, qx, pxb), fmaf(sy, qy, pyb), 2 * k + j); };
+    return rk4_gathered(ask, [](const Gather &G) { return value(G); }, 0.5f, y, dph);
 }
 
 template <bool TAU, bool FORMS>
@@ -1119,6 +1082,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M2 ? 4 : 1)
 constexpr double kTimeTol = 1e-10;
 constexpr int kTimeMaxSteps = 1 << 18;
 
+template <bool FIRST>
 __device__ __forceinline__ void time_rhs(const TraceArgs &a, const double (&y)[7], double (&k)[7]) {
     const double px = (y[0] - a.x0) / a.dx, py = (y[1] - a.y0) / a.dy, pz = (y[2] - a.z0) / a.dz;
     double g[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1144,7 +1108,9 @@ __device__ __forceinline__ void time_rhs(const TraceArgs &a, const double (&y)[7
     k[3] = g[0] * idz;
     k[4] = g[1] * idz;
     k[5] = g[2] * idz;
-    k[6] = g[3] * idz * sqrt(y[3] * y[3] + y[4] * y[4] + y[5] * y[5]);
+    // U . U, its roundings written out (time_speed2 has the same)
+    const double u = FIRST ? fma(y[3], y[3], __dmul_rn(y[4], y[4])) : fma(y[4], y[4], __dmul_rn(y[3], y[3]));
+    k[6] = g[3] * idz * sqrt(fma(y[5], y[5], u));
 }
 
 // Dormand-Prince 5(4) tableau: stage nodes are implied by the rows; the last
@@ -1175,7 +1141,7 @@ __device__ void trace_time_ray(const TraceArgs &a, int64_t t, int32_t only) {
         const double hi[3] = {a.x0 + (double)a.fx1 * a.dx, a.y0 + (double)a.fy1 * a.dy, a.z0 + (double)a.fz1 * a.dz};
         const double sc[6] = {kTimeTol * a.dx, kTimeTol * a.dy, kTimeTol * a.dz, kTimeTol, kTimeTol, kTimeTol};
         double k[7][7];
-        time_rhs(a, y, k[0]);
+        time_rhs<true>(a, y, k[0]);
         double tau = 0.0, h = hmax;
         int tries = 0;
         while (tau < a.cT) {
@@ -1198,7 +1164,10 @@ __device__ void trace_time_ray(const TraceArgs &a, int64_t t, int32_t only) {
                     for (int j = 0; j < st; ++j) acc = fma(kDPA[st - 1][j], k[j][i], acc);
                     yn[i] = fma(hh, acc, y[i]);
                 }
-                time_rhs(a, yn, k[st]);
+                if (st == 1)
+                    time_rhs<true>(a, yn, k[st]);
+                else
+                    time_rhs<false>(a, yn, k[st]);
             }
             double en = 0.0;  // largest scaled error estimate
 #pragma unroll
