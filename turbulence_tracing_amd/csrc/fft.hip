@@ -787,8 +787,9 @@ __global__ __launch_bounds__(kAnyThreads) __attribute__((amdgpu_waves_per_eu(6, 
     constexpr bool kRows = MODE == kPassX || MODE == kFwdX;
     // Neighbouring columns share the lines that their elements lie in: blocks of
     // neighbouring columns go to one XCD, whose L2 then holds a line for all of
-    // them (a block of 4 moves 32 bytes of each).  Fields of 256 x 1280 x 256 1417 ->
-    // 1000 us, 128 x 4096 x 128 1840 -> 1354, 320^3 380 -> 343.
+    // them (a block of 4 moves 32 bytes of each, one of 4096 points 8).  Fields of
+    // 256 x 1280 x 256 1417 -> 1001 us, 128 x 2048 x 128 701 -> 525, 128 x 4096 x 128
+    // 1840 -> 1347, 320^3 380 -> 343.
     const int64_t block = kRows || gridDim.y > 1 ? (int64_t)blockIdx.y * gridDim.x + blockIdx.x
                                                  : tt::xcd_block((int)blockIdx.x, (int)gridDim.x);
     const int64_t first = block * PB;

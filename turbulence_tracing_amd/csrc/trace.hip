@@ -1222,7 +1222,10 @@ __device__ void trace_time_ray(const TraceArgs &a, int64_t t, int32_t only) {
 // Measured on a 101^3 liner that turns every ray back (1190 tries a ray): 16000
 // rays 7.25 -> 2.91 ms, 20000 (some SIMDs with two waves) 7.26 -> 4.63, 30000
 // 7.3 -> 4.8, 40000 7.35 -> 7.0, 100000 13.4 -> 15.3.  So up to kTimeQuadRays,
-// two waves on each of the 1024 SIMDs; one lane a ray beyond.
+// two waves on each of the 1024 SIMDs; one lane a ray beyond, where a third wave a
+// SIMD leaves little of the gain and a fourth none.  The rule goes by the rays of
+// the call, not by those of the status asked for, whose number the host does not
+// know: a few turning rays of a large set take one lane each.
 constexpr int64_t kTimeQuadRays = 32768;
 
 // v of lanes A, B, C, D of each quad, in its lanes 0 to 3
