@@ -253,7 +253,7 @@ def main_ensemble(args):
     """48 realisations of uneven size (grids from {128, 192, 256, 384}^3,
     anisotropic power-law spectra, 2-20% RMS, mean ne 1e23-1e25, 2e5-2e6 rays
     each), every stage of a step (fields, gradients, beams, ray orders, one
-    persistent batched trace, detectors) captured as one HIP graph with the
+    batched trace, detectors) captured as one HIP graph with the
     autotuned launch shape.  A step is one graph replay."""
     import torch
     from turbulence_tracing_amd.ensemble import Ensemble, draw_members

@@ -664,11 +664,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MODE =
 // R) once for kP pencils, so (with kQ = 4) 8 complex products go with 5 LDS
 // reads.  The terms are added in order of r: the same bits as one output per
 // thread with two reads a term, as which it was bound by LDS (201^3 = 3 x 67:
-// 1610 us, here 320; 257^3 5700, here 1730); now it is bound by the products'
+// 1610 us, here 289; 257^3 5700, here 1730); now it is bound by the products'
 // issue.  (With the inputs folded by the symmetry of the factors, on
 // v_mfma_f32_16x16x4_f32, they took 162 and 492 us, but sums in that order move
 // the field's rounding: its sum of squares by more than 1e-9.)  Lengths without
-// such a factor gain from the rest: 300^3 630 -> 330 us, 64^3 87 -> 22 us.
+// such a factor gain from the rest: 300^3 620 -> 317 us, 64^3 85 -> 17 us.
 // 512 threads a block: with 256, 300^3 took 457 us.  Six waves a SIMD: left to
 // itself the compiler takes more registers and 201^3 took 350.
 constexpr int kAnyThreads = 512;
