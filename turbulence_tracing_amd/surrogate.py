@@ -368,7 +368,9 @@ class Surrogate:
         for ep in range(epochs):
             perm = torch.randperm(N, generator=gen, device=self.device)
             loss.zero_()
-            # taken anew each epoch: `log` may load weights or replace the network between two
+            # taken anew each epoch (`log` may load weights or replace the network
+            # between two), after the last one's workspace is given back
+            fused = None
             fused = self._fused_step(X, target, batch, wd) if N >= batch else None
             for b in range(N // batch):
                 idx = perm[b * batch:(b + 1) * batch]
