@@ -401,9 +401,10 @@ extern "C" int tt_detect(const tt_detector *dets, int32_t ndet, const double *rf
             w.ndet = count[g];
             std::copy(a.d + k, a.d + k + count[g], w.d);
             w.d[0].again = 0;
-            // resident at once, each with as many rays as bins to add at least
+            // resident at once, each with as many rays as bins to add at least, and with
+            // 1024, so that fewer partial sums of weights meet in a bin than by windows
             const int64_t blocks = std::min<int64_t>(256 * std::min(4, kWholeBins * 5 / 2 / group[g]),
-                                                     tt::ceil_div(n, (int64_t)std::max(kDetBlock, group[g])));
+                                                     tt::ceil_div(n, (int64_t)std::max(2 * kDetBlock, group[g])));
             hipLaunchKernelGGL(detect_whole_kernel, dim3((unsigned)blocks), dim3(kDetBlock),
                                (size_t)group[g] * sizeof(uint32_t), tt::as_stream(stream), w, group[g]);
             TT_LAUNCH_CHECK("tt_detect launch");
